@@ -137,11 +137,24 @@ int hh_prefill_attn_mfma_launch(int hd, const float* QB, const float* k_cache, c
 // gate: qwen35 gated attention's projection rows (gate_row floats apart), or null;
 // kv_q8: the caches hold Q8_0 rows (quantized on write, dequantized on load)
 
-// Batched Q8_0 GEMM on int8 MFMA (prefill): out[s*n + r], K % 128 == 0, activations
+// Batched GEMM of Q8_0 weights on int8 MFMA: out[s*n + r], K % 128 == 0, activations
 // split (int8 xq[seq][K], f32 xd[seq][K/32]); hh_q8_split_launch converts standard Q8_0 rows.
-int hh_gemm_launch(int fmt, const uint8_t* w, int n, int K, const int8_t* xq, const float* xd, int seq, float* out,
+int hh_gemm_launch(const uint8_t* w, int n, int K, const int8_t* xq, const float* xd, int seq, float* out,
                    hipStream_t s);
 int hh_q8_split_launch(const uint8_t* x, int64_t nblocks, int8_t* xq, float* xd, hipStream_t s);
+// The same product for the 1- and 2-bit formats (Q1, Q2, PT) on the f8f6f4 matrix
+// instructions (hh_gemm_f4.hip), activations in tiles of 32 tokens x 128 columns
+// made for the weight format: hh_act_tiles_launch from standard Q8_0 rows (x), or
+// from xq / xd (x null).
+constexpr int HH_ACT_TILE_BYTES = 6656;
+size_t hh_act_tiles_bytes(int K, int seq);
+int hh_act_tiles_launch(int fmt, const uint8_t* x, const int8_t* xq, const float* xd, int K, int seq, uint8_t* tiles,
+                        hipStream_t s);
+// wtiles: hh_gemm_f4_wbytes(n, K, seq) bytes of scratch (null: not used, slower from
+// 256 tokens on)
+size_t hh_gemm_f4_wbytes(int n, int K, int seq);
+int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* tiles, int seq, uint8_t* wtiles,
+                      float* out, hipStream_t s);
 
 int hh_quantize_launch(const float* x, int64_t n, uint8_t* out, hipStream_t s);
 int hh_dequant_launch(int type, const void* w, int64_t n, float* out, hipStream_t s);

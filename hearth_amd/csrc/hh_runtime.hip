@@ -560,6 +560,8 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   int n_in_max = 0;
   for (const Layer& L : m->layers) n_in_max = std::max(n_in_max, L.n_in);
   const int kmax = std::max(std::max(d, F), std::max(nq, vdim));
+  const size_t wt_max = std::max(std::max(hh_gemm_f4_wbytes(n_in_max, d, S), hh_gemm_f4_wbytes(2 * F, d, S)),
+                                 std::max(hh_gemm_f4_wbytes(d, F, S), hh_gemm_f4_wbytes(d, std::max(nq, vdim), S)));
   // scratch layout
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align256(off + bytes); return o; };
@@ -572,6 +574,7 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
                oGAB = take(hyb ? (size_t)S * 2 * c.ssm_n_v_heads * 4 : 0),
                oGDEC = take(hyb ? (size_t)S * c.ssm_n_v_heads * 4 : 0), oGO = take(hyb ? (size_t)S * vdim * 4 : 0),
                oRot = take(c.had_block > 0 ? (size_t)S * std::max(std::max(vdim, nq), F) * 4 : 0),
+               oAct = take(hh_act_tiles_bytes(kmax, S)), oWt = take(wt_max),
                oChunk = take(hyb && chunked ? hh_gdn_chunk_scratch_bytes(c.ssm_n_v_heads, S) : 0);
   if (off > m->pf_cap) {
     if (m->pf_buf) HIP_TRY(hipFree(m->pf_buf));
@@ -584,6 +587,7 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   float* H = (float*)(B + oH);
   int8_t* Xq = (int8_t*)(B + oXq);
   float* Xd = (float*)(B + oXd);
+  uint8_t* Act = B + oAct;
   float* QKV = (float*)(B + oQKV);
   float* QB = (float*)(B + oQB);
   float* T = (float*)(B + oT);
@@ -599,6 +603,10 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
     if (had) return hh_rot_q8_rows_launch(H, w, c.eps, d, S, signs_of(m, d), c.had_block, 0, 0, Xq, Xd, s);
     return hh_norm_q8_rows_launch(H, w, c.eps, d, S, Xq, Xd, s);
   };
+  auto gemm = [&](const uint8_t* w, int n, int K, float* out) -> int {
+    const int rc = hh_act_tiles_launch(m->wfmt, nullptr, Xq, Xd, K, S, Act, s);
+    return rc ? rc : hh_gemm_f4_launch(m->wfmt, w, n, K, Act, S, wt_max ? B + oWt : nullptr, out, s);
+  };
   KTRY(hh_embed_rows_launch(c.head_type, m->token_embd->d, d, toks, S, H, latent ? signs_of(m, d) : nullptr,
                             latent ? c.had_block : 0, s));
   for (int li = 0; li < c.n_layers; ++li) {
@@ -611,7 +619,7 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
       if (li > 0) KTRY(hh_add_rows_launch(H, T, (int64_t)S * d, s));
       KTRY(norm_rows(L.attn_norm));
     }
-    KTRY(hh_gemm_launch(m->wfmt, L.w_in, L.n_in, d, Xq, Xd, S, QKV, s));
+    KTRY(gemm(L.w_in, L.n_in, d, QKV));
     int k_out;
     if (L.gdn) {
       GdnArgs ga{};
@@ -665,17 +673,17 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
         KTRY(hh_rot_q8_rows_launch(Rot, nullptr, 0.0f, nq, S, signs_of(m, nq), c.had_block, 0, 0, Xq, Xd, s));
       k_out = nq;
     }
-    KTRY(hh_gemm_launch(m->wfmt, L.w_out, d, k_out, Xq, Xd, S, T, s));
+    KTRY(gemm(L.w_out, d, k_out, T));
     if (!had) {
       KTRY(hh_add_norm_q8_rows_launch(H, T, L.ffn_norm, c.eps, d, S, Xq, Xd, s));
     } else {
       KTRY(hh_add_rows_launch(H, T, (int64_t)S * d, s));
       KTRY(norm_rows(L.ffn_norm));
     }
-    KTRY(hh_gemm_launch(m->wfmt, L.w_gu, 2 * F, d, Xq, Xd, S, GU, s));
+    KTRY(gemm(L.w_gu, 2 * F, d, GU));
     KTRY(hh_silu_q8_rows_launch(GU, F, S, Xq, Xd, Rot, s));
     if (had) KTRY(hh_rot_q8_rows_launch(Rot, nullptr, 0.0f, F, S, signs_of(m, F), c.had_block, 0, 0, Xq, Xd, s));
-    KTRY(hh_gemm_launch(m->wfmt, L.w_down, d, F, Xq, Xd, S, T, s));
+    KTRY(gemm(L.w_down, d, F, T));
     // the residual add: fused into the next layer's input norm, plain after the last
     if (li + 1 == c.n_layers) KTRY(hh_add_rows_launch(H, T, (int64_t)S * d, s));
   }
@@ -844,20 +852,36 @@ int hh_gemm_q8(hh_ctx* c, int type, const void* w, int64_t n_rows, int64_t n_col
   if (n_rows <= 0 || n_rows > (1ll << 30) || seq_len <= 0 || seq_len > (1ll << 24))
     return fail(HH_ERR_DIM, "bad n_rows or seq_len");
   if ((n_rows + 63) / 64 > 2147483647ll || (seq_len + 63) / 64 > 65535) return fail(HH_ERR_DIM, "grid too large");
-  // the GEMM reads its activations as int8 rows plus f32 block scales
-  const size_t nq = (size_t)seq_len * n_cols, need = align256(nq) + nq / 32 * 4;
-  if (c->gemm_scratch_bytes < need) {
+  // scratch, grown on demand: activation tiles and, for many tokens, expanded
+  // weights (1- and 2-bit formats), or int8 rows plus f32 block scales (Q8_0)
+  const size_t nq = (size_t)seq_len * n_cols;
+  const size_t act = align256(fmt == FMT_Q8 ? nq : hh_act_tiles_bytes((int)n_cols, (int)seq_len));
+  const size_t extra = fmt == FMT_Q8 ? nq / 32 * 4 : hh_gemm_f4_wbytes((int)n_rows, (int)n_cols, (int)seq_len);
+  if (c->gemm_scratch_bytes < act + extra) {
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (c->gemm_scratch) HIP_TRY(hipFree(c->gemm_scratch));
     c->gemm_scratch = nullptr;
     c->gemm_scratch_bytes = 0;
-    HIP_TRY(hipMalloc(&c->gemm_scratch, need));
-    c->gemm_scratch_bytes = need;
+    size_t got = act + extra;
+    if (hipMalloc(&c->gemm_scratch, got) != hipSuccess) {
+      c->gemm_scratch = nullptr;
+      (void)hipGetLastError();
+      got = fmt == FMT_Q8 ? got : act;   // the product runs without the expanded weights too
+      HIP_TRY(hipMalloc(&c->gemm_scratch, got));
+    }
+    c->gemm_scratch_bytes = got;
   }
-  int8_t* xq = (int8_t*)c->gemm_scratch;
-  float* xd = (float*)((char*)c->gemm_scratch + align256(nq));
+  uint8_t* buf = (uint8_t*)c->gemm_scratch;
+  if (fmt != FMT_Q8) {
+    KTRY(hh_act_tiles_launch(fmt, xq8, nullptr, nullptr, (int)n_cols, (int)seq_len, buf, c->stream));
+    KTRY(hh_gemm_f4_launch(fmt, (const uint8_t*)w, (int)n_rows, (int)n_cols, buf, (int)seq_len,
+                           extra && c->gemm_scratch_bytes >= act + extra ? buf + act : nullptr, out, c->stream));
+    return HH_OK;
+  }
+  int8_t* xq = (int8_t*)buf;
+  float* xd = (float*)(buf + act);
   KTRY(hh_q8_split_launch(xq8, (int64_t)(nq / 32), xq, xd, c->stream));
-  KTRY(hh_gemm_launch(fmt, (const uint8_t*)w, (int)n_rows, (int)n_cols, xq, xd, (int)seq_len, out, c->stream));
+  KTRY(hh_gemm_launch((const uint8_t*)w, (int)n_rows, (int)n_cols, xq, xd, (int)seq_len, out, c->stream));
   return HH_OK;
 }
 

@@ -251,6 +251,34 @@ def test_gemm_bit_exact_vs_per_token_dot(ctx, oracle, t, n, k, seq):
         assert np.array_equal(got[s], want), s
 
 
+@pytest.mark.parametrize("t", [41, 42, 143])
+@pytest.mark.parametrize("n,k,seq", [
+    (1, 128, 1), (33, 256, 32), (127, 384, 33), (257, 640, 255),      # straight from the blocks
+    (31, 128, 256), (257, 256, 257), (130, 384, 300), (512, 1024, 511),  # expanded, 128 x 64 by 8 waves; 1..8 steps
+    (4096, 128, 1024), (4095, 256, 1000),                             # 128 x 64 by 4 waves
+    (6144, 128, 2048), (4096, 384, 2048)])                            # 128 x 128 and 256 x 128
+def test_gemm_tiles_bit_exact(ctx, oracle, t, n, k, seq):
+    """Every tile shape of the 1- and 2-bit GEMM, at row, token and step counts around
+    its edges, on arbitrary codes, scales and activation bytes (-128 included): equal to
+    the scalar DotFn bit for bit on the tokens at tile edges."""
+    print(f"gemm tiles t={t} n={n} k={k} seq={seq}", flush=True)
+    rng = np.random.default_rng(n + k + seq + t)
+    w = _random_weights(t, n, k, rng)
+    xq = rng.integers(0, 256, (seq * k // 32, 34), dtype=np.uint8)
+    sc = (rng.uniform(0, 2, len(xq)) * 10.0 ** rng.integers(-3, 2, len(xq))).astype(np.float16).view(np.uint16)
+    xq[:, 0], xq[:, 1] = sc & 0xFF, sc >> 8
+    xq = xq.reshape(seq, -1)
+    xq[seq - 1].reshape(-1, 34)[:, 2:] = 128
+    out = torch.full((seq * n + 64,), 7.0, dtype=torch.float32, device="cuda")
+    ctx.gemm_q8(t, dev(w), n, k, dev(xq.reshape(-1)), seq, out)
+    got = host(out)
+    assert np.all(got[seq * n:] == 7.0)
+    got = got[:seq * n].reshape(seq, n)
+    for s in sorted({v for e in range(0, seq + 32, 32) for v in (e - 1, e) if 0 <= v < seq and (seq < 600 or e % 512 == 0)}
+                    | {seq - 1}):
+        assert np.array_equal(got[s], oracle.gemv(t, w, n, k, xq[s])), s
+
+
 def test_gemm_errors(ctx):
     from hearth_amd import HHError
     w = torch.zeros(4096, dtype=torch.uint8, device="cuda")
