@@ -190,45 +190,9 @@ HH_DEV float4 slice_rope(float4 x, float4 sn, float4 cs, int c4, int rope_dim) {
 // the all-lanes butterfly x_l + x_(l^O) at that level, so the result for
 // value k is the butterfly sum with offsets LPR/2, ..., 1.  On return lane l
 // holds value k = (l % LPR) >> log2(LPR / NV).
-// Lanes hand over their values in a lane-dependent register order: register
-// r of lane l holds value r ^ rs_perm<NV, LPR / 2>(l).  At each level below
-// offset 16 every lane then keeps registers [0, N/2) and sends [N/2, N): a
-// lane whose offset bit is set holds the upper half in the lower registers,
-// and its partner's upper registers hold that same half, so each kept sum is
-// the same pair of values, added in the same order, with no per-lane select.
-// (The permlane swaps of the offsets 16 and 32 pair registers r and r + N/2
-// across the lanes themselves.)
-template <int N, int O> HH_DEV int rs_perm(int lane) {
-  if constexpr (N > 1) return ((O < 16 && (lane & O)) ? N / 2 : 0) ^ rs_perm<N / 2, O / 2>(lane);
-  else return 0;
-}
-template <int N, int O> struct ReduceScatter {
-  static HH_DEV float run(float* v) {
-    if constexpr (N > 1) {
-      static_assert(O > 0, "more values than lanes");
-#pragma unroll
-      for (int k = 0; k < N / 2; ++k) {
-        if constexpr (O >= 16) v[k] = swap_pair_sum<O>(v[k], v[k + N / 2]);
-        else v[k] = v[k] + xor_lane<O>(v[k + N / 2]);
-      }
-      return ReduceScatter<N / 2, O / 2>::run(v);
-    } else {
-      float x = v[0];
-      if constexpr (O >= 32) x += xor_lane<32>(x);
-      if constexpr (O >= 16) x += xor_lane<16>(x);
-      if constexpr (O >= 8) x += xor_lane<8>(x);
-      if constexpr (O >= 4) x += xor_lane<4>(x);
-      if constexpr (O >= 2) x += xor_lane<2>(x);
-      if constexpr (O >= 1) x += xor_lane<1>(x);
-      return x;
-    }
-  }
-};
-
-// The same butterfly sum with values in the natural register order: lanes
-// whose offset bit is set keep the upper half, chosen per lane.  The decode
-// split uses it: its one pass is latency-bound, and the permuted order's
-// extra K addressing and q swaps cost more there than the selects.
+// At the offsets below 16 the lanes whose offset bit is set keep the upper half,
+// chosen per lane; the permlane swaps of 16 and 32 pair registers k and k + N/2
+// across the lanes themselves.
 template <int N, int O> struct ReduceScatterSel {
   static HH_DEV float run(float* v, int lane) {
     if constexpr (N > 1) {
@@ -953,207 +917,371 @@ __global__ __launch_bounds__(512) void k_prefill_qk(const float* __restrict__ QK
   }
 }
 
-// Prefill attention, split pass: workgroup (chunk c, kv head, token tile)
-// holds K/V rows of chunk c in registers exactly as k_attn_split does and
-// runs the decode arithmetic (scores, chunk softmax, P.V and their reduction
-// order) once per token of the tile whose position reaches the chunk, NTOK
-// tokens per pass.  GMAX bounds the query heads per kv head (registers).
-// Partials: PO[((sl*n_kv + kvh)*n_chunks + c)*G + h][HD], PML likewise x2.
-template <int HD, int NTA, bool KV8, int GMAX, int NTOK, int GT, int C>
-__global__ __launch_bounds__(NTA) void k_attn_prefill_split(const float* __restrict__ QB, const float* __restrict__ k_cache,
-                                                            const float* __restrict__ v_cache, int n_heads, int n_kv,
-                                                            int max_seq, int pos0, int S, int t0, int TT, int n_chunks,
-                                                            float* __restrict__ PO, float* __restrict__ PML) {
-  constexpr int LPR = HD / 4, RPI = NTA / LPR, NR = C / RPI, NW = NTA / 64;
-  extern __shared__ __align__(16) float sm[];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int c = blockIdx.x, kvh = blockIdx.y, G = GT > 0 ? GT : n_heads / n_kv;
-  const int sl0 = blockIdx.z * TT, sl1 = min(sl0 + TT, S - t0);   // tile-launch-relative tokens
-  const int p0 = c * C;
-  const int np_max = min(C, pos0 + t0 + sl1 - p0);
-  if (sl0 >= sl1 || np_max <= 0) return;
-  const int sub = tid / LPR, cc = tid % LPR;
-  float* sc = sm;                          // NTOK * G * C
-  float* ml = sc + NTOK * G * C;           // NTOK * 2 * G (+pad)
-  float* red = ml + ((NTOK * 2 * G + 4 + 3) & ~3);   // NTOK * NW waves * 4 heads * HD (16-byte aligned)
-  const size_t hstride = (size_t)max_seq * HD;
-  const float* kg = k_cache + (size_t)kvh * hstride + 4 * cc;
-  const float* vg = v_cache + (size_t)kvh * hstride + 4 * cc;
-  // K rows and q heads in the reduce-scatter's register order
-  // (ReduceScatter): K register i holds row (i ^ pi) * RPI + sub, q register
-  // h of a group of four head (h ^ ph); V rows stay in order (the P.V chain
-  // runs over i).  The q rows arrive normalized and rotated, so no step here
-  // needs the lanes of a row on one head.
-  constexpr int NV = 4 * NR;
-  const int rsp = rs_perm<NV, LPR / 2>(lane), pi = rsp % NR, ph = rsp / NR;
-  float4 kr[NR], vr[NR];
-  // every K row before the V rows (the scores need only K)
+// ---------------------------------------------------------------------------
+// Prefill attention, split pass: the decode split's arithmetic (k_attn_split) for
+// tiles of 16 prompt tokens on the fp32 matrix instructions.
+//
+// v_mfma_f32_16x16x4_f32 is, per output, the chain fma(a3, b3, fma(a2, b2,
+// fma(a1, b1, fma(a0, b0, c)))) with each step rounded (checked on the device bit
+// for bit, subnormals included).  Both chains of the decode split have that form:
+// a score's partial over the 4 dims of a lane's slice, and P.V over the rows
+// i = 4u .. 4u + 3 of a row group.  What is left for the vector unit are the
+// decode split's sums between lanes and waves, here sums of result registers in
+// the same order:
+//   score = node(0, 1), node(c, O) = node(c, 2 O) + node(c + O, 2 O), the slice
+//   partials at O = hd / 4 (the reduce-scatter's descending butterfly);
+//   o = the pairwise tree over the row groups.
+// So every partial equals the decode split's bit for bit.  Matrix and vector pipe
+// are about level (per wave, 16 queries and 64-position chunk 64 products of 32
+// cycles and about 500 vector operations of 4).  With the dots on the vector pipe,
+// split + merge of an 8B layer (32/8 heads x 128) took 252 us for 777 tokens at
+// position 250 and 1.79 ms for 2048 at 0; here 160 us and 0.66 ms, 0.13 ms of that
+// the merge.
+//
+// Workgroup (kv head, chunk, tpw tiles of 16 tokens), NWV waves.  Position j = i * RPI
+// + sub of the chunk (as in k_attn_split), i = 4u + g: lane group g = lane / 16 holds
+// the rows with i % 4 = g, its value v = u * RPI + sub.  Wave w holds, in registers,
+// the K rows of values 4p .. 4p + 3 (p = w % NP: one score tile of 16 positions) and
+// the V columns of its EW dim tiles.  Per token tile and HB query heads: each wave
+// computes its score tile of every head (q from LDS, the next ones copied there
+// meanwhile), the maxima and then the exponentials meet in LDS, and each wave runs
+// P.V for its dim tiles.  A score register is (lane % 16 = token, value 4p + r), so
+// the exponentials a lane reads back are exactly its B operand of P.V.
+// ---------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// 4x4 transpose across the lane groups: in, a[e] of group g = M[g][e]; out, a[r] of
+// group g = M[r][g].
+HH_DEV void transpose_groups(float a[4]) {
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const int jk = (i ^ pi) * RPI + sub;
-    kr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if constexpr (KV8) {
-      const size_t r = (size_t)kvh * max_seq + p0;
-      if (jk < np_max) kr[i] = KvQ8(const_cast<float*>(k_cache), n_kv, max_seq, HD).load(r + jk, HD, cc);
-    } else {
-      if (jk < np_max) kr[i] = *(const float4*)(kg + (size_t)(p0 + jk) * HD);
-    }
+  for (int i = 0; i < 2; ++i) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[i]), __float_as_uint(a[i + 2]), false, false);
+    a[i] = __uint_as_float(r[0]);
+    a[i + 2] = __uint_as_float(r[1]);
   }
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const int j = i * RPI + sub;
-    vr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if constexpr (KV8) {
-      const size_t r = (size_t)kvh * max_seq + p0;
-      if (j < np_max) vr[i] = KvQ8(const_cast<float*>(v_cache), n_kv, max_seq, HD).load(r + j, HD, cc);
-    } else {
-      if (j < np_max) vr[i] = *(const float4*)(vg + (size_t)(p0 + j) * HD);
-    }
+  for (int i = 0; i < 4; i += 2) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[i]), __float_as_uint(a[i + 1]), false, false);
+    a[i] = __uint_as_float(r[0]);
+    a[i + 1] = __uint_as_float(r[1]);
   }
+}
+
+HH_DEV f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// Eight products, and between them the pairwise tree ((p0 + p1) + (p2 + p3)) + .. of
+// the eight before: the matrix pipe works while the sums run.
+#define HH_KEEP_ORDER() __builtin_amdgcn_sched_barrier(0x74)   // global memory and scalar operations may cross
+template <class F> HH_DEV f32x4 products8(f32x4 (&d)[8], const f32x4 (&p)[8], F product) {
+  d[0] = product(0); HH_KEEP_ORDER();
+  f32x4 a = p[0] + p[1]; HH_KEEP_ORDER();
+  d[1] = product(1); HH_KEEP_ORDER();
+  f32x4 b = p[2] + p[3]; HH_KEEP_ORDER();
+  d[2] = product(2); HH_KEEP_ORDER();
+  a = a + b; HH_KEEP_ORDER();
+  d[3] = product(3); HH_KEEP_ORDER();
+  b = p[4] + p[5]; HH_KEEP_ORDER();
+  d[4] = product(4); HH_KEEP_ORDER();
+  f32x4 c = p[6] + p[7]; HH_KEEP_ORDER();
+  d[5] = product(5); HH_KEEP_ORDER();
+  b = b + c; HH_KEEP_ORDER();
+  d[6] = product(6); HH_KEEP_ORDER();
+  a = a + b; HH_KEEP_ORDER();
+  d[7] = product(7); HH_KEEP_ORDER();
+  return a;
+}
+HH_DEV f32x4 tree8(const f32x4 (&p)[8]) {
+  return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+}
+
+// node(0, 1) over NS slice products (NS 32 or 64): groups node(c, NS / 8) of eight,
+// then the levels above.  q(c): the query's value of slice c, read one group ahead.
+template <int NS, class Q> HH_DEV f32x4 score_tree(const float (&k)[NS], Q q) {
+  constexpr int NG = NS / 8;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 d[2][8], s[4];   // s: the left siblings of the levels above, as they are made
+  float qv[2][8];
+  auto up = [&](int j, f32x4 v) {   // group j's node joins them
+    int l = 0;
+#pragma unroll
+    for (; l < 3; ++l) {
+      if (!((j >> l) & 1)) break;
+      v = s[l] + v;
+    }
+    s[l] = v;
+  };
+  auto order = [](int i) { return NG == 4 ? (i & 1) * 2 + (i >> 1) : (i & 1) * 4 + (i & 2) + (i >> 2); };   // bit reversal
+  auto leaf = [](int c, int i) { return c + (i & 1) * (NS / 2) + ((i >> 1) & 1) * (NS / 4) + (i >> 2) * (NS / 8); };
+#pragma unroll
+  for (int i = 0; i < 8; ++i) qv[0][i] = q(leaf(0, i));
+#pragma unroll
+  for (int i = 0; i < 8; ++i) qv[1][i] = q(leaf(order(1), i));
+  HH_KEEP_ORDER();
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    d[0][i] = mfma4(k[leaf(0, i)], qv[0][i], zero);
+    HH_KEEP_ORDER();
+  }
+#pragma unroll
+  for (int j = 1; j < NG; ++j) {
+    const int c = order(j);
+    if (j + 1 < NG) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) qv[(j + 1) & 1][i] = q(leaf(order(j + 1), i));
+    }
+    up(j - 1, products8(d[j & 1], d[(j - 1) & 1], [&](int i) { return mfma4(k[leaf(c, i)], qv[j & 1][i], zero); }));
+  }
+  up(NG - 1, tree8(d[(NG - 1) & 1]));
+  return s[NG == 4 ? 2 : 3];
+}
+
+// The pairwise trees over the RPI row groups (8 or 16) of EW dim tiles; NU chained
+// products per row group.
+template <int EW, int CV, int RPI, int NU> HH_DEV void pv_trees(const float (&v)[EW][CV], const float (&e)[CV], f32x4 (&o)[EW]) {
+  constexpr int NG = EW * RPI / 8;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 d[2][8], s[NG];
+  auto first = [&](int j, int i) {
+    const int t = j * 8 / RPI, sub = j * 8 % RPI + i;
+    return mfma4(v[t][sub], e[sub], zero);
+  };
+  auto chain = [&](int j) {
+    if constexpr (NU == 2) {
+      const int t = j * 8 / RPI;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int sub = RPI + j * 8 % RPI + i;
+        d[j & 1][i] = mfma4(v[t][sub], e[sub], d[j & 1][i]);
+      }
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    d[0][i] = first(0, i);
+    HH_KEEP_ORDER();
+  }
+  chain(0);
+#pragma unroll
+  for (int j = 1; j < NG; ++j) {
+    s[j - 1] = products8(d[j & 1], d[(j - 1) & 1], [&](int i) { return first(j, i); });
+    chain(j);
+  }
+  s[NG - 1] = tree8(d[(NG - 1) & 1]);
+#pragma unroll
+  for (int t = 0; t < EW; ++t) o[t] = RPI == 16 ? s[2 * t] + s[2 * t + (RPI == 16 ? 1 : 0)] : s[t];
+}
+
+// Partials: PO[((sl*n_kv + kvh)*n_chunks + c)*G + h][HD], PML likewise x2, for the
+// tokens sl of [t0, t0 + n) whose position reaches chunk c.
+template <int HD, bool KV8, int NWV, int C>
+__global__ __launch_bounds__(64 * NWV, 2) void k_attn_prefill_split(const float* __restrict__ QB,
+                                                                    const float* __restrict__ k_cache,
+                                                                    const float* __restrict__ v_cache, int n_heads,
+                                                                    int n_kv, int max_seq, int pos0, int t0, int n,
+                                                                    int nc, int tpw, int n_chunks,
+                                                                    float* __restrict__ PO, float* __restrict__ PML) {
+  constexpr int NS = HD / 4, RPI = ATTN_NT / NS, NU = C / RPI / 4, CV = C / 4;   // CV: values per lane
+  constexpr int NP = C / 16, QS = NWV / NP, EW = HD / 16 / NWV, HB = HD == 128 ? 4 : 2, ES = CV + 4;
+  static_assert(QS * NP == NWV && (QS == 1 || QS == 2) && (EW == 1 || EW == 2 || EW == 4), "wave split");
+  constexpr int QL = HB * 16 * HD / 4 / (64 * NWV);   // 16-byte copies of q per lane and batch
+  __shared__ float sm_m[HB][NP][16];
+  __shared__ __align__(16) float sm_e[HB][64][ES];   // [token * 4 + g]; row stride 16 (2 k + 1) bytes: no conflicts
+  // q, 1 KB copies: two tokens' units interleaved (hd 128) or one token (hd 256), padded
+  // so that 16 tokens' reads of one slice fall on 64 banks
+  constexpr int QP = HD == 128 ? 264 : 260;
+  __shared__ __align__(16) float sm_q[HB * 16 * HD / 256 * QP];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
+  // kv head fastest: with the round-robin dispatch a head's K and V stay in one XCD's
+  // L2; the last tokens, which reach every chunk, first
+  const int kvh = blockIdx.x % n_kv, rest = blockIdx.x / n_kv, c = rest % nc, z = gridDim.x / n_kv / nc - 1 - rest / nc;
+  const int G = n_heads / n_kv, p0 = c * C;
+  const int p = wid % NP, qs = wid / NP, dim0 = wid * 16 * EW + EW * l16;   // dim tile e: dims 16 EW wid + EW d + e
+  const float* kg = k_cache + (size_t)kvh * max_seq * HD;
+  const float* vg = v_cache + (size_t)kvh * max_seq * HD;
+  const size_t kv_row = (size_t)kvh * max_seq + p0;
   const float inv_sqrt = 1.0f / sqrtf((float)HD);
-  constexpr int KSH = (LPR == 64 ? 6 : 5) - (NV == 32 ? 5 : NV == 16 ? 4 : 3);
-  // NTOK tokens per pass (each with the decode arithmetic of one token): their
-  // softmax rows spread over all waves and they share the barriers.  Tokens
-  // before the first whose position reaches the chunk skip it.
-  const int sl_first = max(sl0, p0 - pos0 - t0);
-  for (int sl = sl_first; sl < sl1; sl += NTOK) {
-    const int nt = min(NTOK, sl1 - sl);
+  // first tile whose last token reaches the chunk
+  int ta = z * tpw * 16;
+  const int tend = min(ta + tpw * 16, n);
+  while (ta < tend && pos0 + t0 + min(ta + 16, n) <= p0) ta += 16;
+  if (ta >= tend) return;
+  // straight from memory to LDS, 1 KB per wave and copy: the heads hb .. hb + HB - 1 of
+  // the tile at tb, past the end clamped
+  auto copy_q = [&](int tb, int hb) {
 #pragma unroll
-    for (int u = 0; u < NTOK; ++u) {
-      if (u >= nt) break;   // uniform
-      const int s = t0 + sl + u, np = min(C, pos0 + s + 1 - p0);
-      float4 q4[GMAX];
-#pragma unroll
-      for (int h = 0; h < GMAX; ++h) {
-        q4[h] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if ((h & ~3) < G) {
-          const int hs = (h & ~3) | ((h & 3) ^ ph);
-          const float* qp = QB + (size_t)s * n_heads * HD + (size_t)(kvh * G + hs) * HD + 4 * cc;
-          q4[h] = *(const float4*)(hs < G ? qp : attn_zero_row);
-        }
-      }
-      float* scu = sc + u * G * C;
-#pragma unroll
-      for (int hg = 0; hg < GMAX; hg += 4) {
-        if (hg >= G) break;
-        float v[NV];
-#pragma unroll
-        for (int hh = 0; hh < 4; ++hh) {
-          const float4 qq = hg + hh < GMAX ? q4[hg + hh] : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-          for (int i = 0; i < NR; ++i) {
-            float pp = qq.x * kr[i].x;
-            pp = fmaf(qq.y, kr[i].y, pp);
-            pp = fmaf(qq.z, kr[i].z, pp);
-            pp = fmaf(qq.w, kr[i].w, pp);
-            v[hh * NR + i] = pp;
-          }
-        }
-        const float r = ReduceScatter<NV, LPR / 2>::run(v);
-        const int k = (lane & (LPR - 1)) >> KSH;
-        const int h = hg + k / NR, j = (k % NR) * RPI + sub;
-        if (h < G && (lane & ((1 << KSH) - 1)) == 0) scu[h * C + j] = (j < np) ? r * inv_sqrt : -INFINITY;
-      }
+    for (int i = 0; i < QL; ++i) {
+      const int f = __builtin_amdgcn_readfirstlane(wid) + NWV * i;
+      const int row = HD == 128 ? 2 * f + (lane & 1) : f, u = HD == 128 ? lane >> 1 : lane, t = row % 16, h = row / 16;
+      const float* src = QB + ((size_t)(t0 + min(tb + t, n - 1)) * n_heads + (size_t)kvh * G + min(hb + h, G - 1)) * HD +
+                         4 * u;
+      __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) const void*)src,
+                                       (__attribute__((address_space(3))) void*)(sm_q + f * QP), 16, 0, 0);
     }
-    __syncthreads();
-    for (int pr = wid; pr < nt * G; pr += NW) {
-      const int u = pr / G, h = pr % G;
-      const int np = min(C, pos0 + t0 + sl + u + 1 - p0);
-      float* row = sc + (u * G + h) * C;
-      if constexpr (C <= 64) {
-        float x = lane < C ? row[lane] : -INFINITY;
-        float m = wave_max_nonan(x);
-        float e = (lane < np) ? hx_exp(x - m) : 0.0f;
-        float l = wave_sum(e);
-        if (lane < C) row[lane] = e;
-        if (lane == 0) { ml[(u * G + h) * 2] = m; ml[(u * G + h) * 2 + 1] = l; }
-      } else {   // C = 128, as the decode split
-        const float x0 = row[lane], x1 = row[64 + lane];
-        const float m = wave_max_nonan(fmaxf(x0, x1));
-        const float e0 = (lane < np) ? hx_exp(x0 - m) : 0.0f;
-        const float e1 = (64 + lane < np) ? hx_exp(x1 - m) : 0.0f;
-        const float l = wave_sum(e0 + e1);
-        row[lane] = e0;
-        row[64 + lane] = e1;
-        if (lane == 0) { ml[(u * G + h) * 2] = m; ml[(u * G + h) * 2 + 1] = l; }
-      }
-    }
-    __syncthreads();
-    for (int hg = 0; hg < G; hg += 4) {
+  };
+  auto wait_q = [] { __builtin_amdgcn_s_waitcnt(7 << 4 | 15 << 8); };   // vmcnt(0): this wave's copies have landed
+  copy_q(ta, 0);
+  wait_q();
+  float kr[NS], vr[EW][CV];
+  int have = 0;   // rows held; rows from there on are zeros
+  for (; ta < tend; ta += 16) {
+    const int np_max = min(C, pos0 + t0 + min(ta + 16, n) - p0);
+    if (np_max != have) {
+      have = np_max;
+      // rows past np_max (other tokens' or none) read a row that is there and become zeros
+      const int v0 = 4 * p + (l16 & 3), jk = (4 * (v0 / RPI) + (l16 >> 2)) * RPI + v0 % RPI;
+      const bool kin = jk < np_max;
+      const int jkc = min(jk, np_max - 1);
+      // (every load is issued before the first value is used)
+      const float* kc = kg + (size_t)p0 * HD;
+      const float* vc = vg + (size_t)p0 * HD;
 #pragma unroll
-      for (int u = 0; u < NTOK; ++u) {
-        if (u >= nt) break;
-        float acc[16];
-#pragma unroll
-        for (int hh = 0; hh < 4; ++hh) {
-          float o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
-          if (hg + hh < G) {
-            const float* eh = sc + (u * G + hg + hh) * C + sub;
-#pragma unroll
-            for (int i = 0; i < NR; ++i) {
-              const float e = eh[i * RPI];
-              o0 = fmaf(e, vr[i].x, o0);
-              o1 = fmaf(e, vr[i].y, o1);
-              o2 = fmaf(e, vr[i].z, o2);
-              o3 = fmaf(e, vr[i].w, o3);
-            }
-          }
-          acc[hh * 4 + 0] = o0; acc[hh * 4 + 1] = o1; acc[hh * 4 + 2] = o2; acc[hh * 4 + 3] = o3;
-        }
-        float* redu = red + u * NW * 4 * HD;
-        if constexpr (LPR == 32) {
-          const bool up = (lane & 32) != 0;
-          float xs[8];
-#pragma unroll
-          for (int k = 0; k < 8; ++k) xs[k] = swap_pair_sum<32>(acc[k], acc[k + 8]);
-#pragma unroll
-          for (int g = 0; g < 2; ++g)   // two 16-byte writes per lane, as the decode split
-            *(float4*)(redu + (wid * 4 + g + (up ? 2 : 0)) * HD + 4 * cc) =
-                make_float4(xs[4 * g], xs[4 * g + 1], xs[4 * g + 2], xs[4 * g + 3]);
+      for (int cc = 0; cc < NS / 4; ++cc) {
+        f32x4 x;
+        if constexpr (KV8) {
+          const float4 f = KvQ8(const_cast<float*>(k_cache), n_kv, max_seq, HD).load(kv_row + jkc, HD, 4 * cc + g);
+          x = f32x4{f.x, f.y, f.z, f.w};
         } else {
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            *(float4*)(redu + (wid * 4 + g) * HD + 4 * cc) =
-                make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
+          x = *(const f32x4*)(kc + (uint32_t)(jkc * HD + 16 * cc + 4 * g));
         }
-      }
-      __syncthreads();
-      if constexpr (4 * HD == NTA) {
-        // lane tid owns value r4 = tid of every token u: its partial sits at
-        // a fixed offset from token u's block, one token stride apart
-        const int h = hg + tid / HD;
-        if (h < G) {
-          const size_t tok = (size_t)n_kv * n_chunks * G * HD;
-          float* dst = PO + (((size_t)sl * n_kv + kvh) * n_chunks + c) * G * HD + (size_t)hg * HD + tid;
-          for (int u = 0; u < nt; ++u) {
-            const float* redu = red + u * NW * 4 * HD;
-            float t[NW];
 #pragma unroll
-            for (int w = 0; w < NW; ++w) t[w] = redu[w * 4 * HD + tid];
-            dst[u * tok] = pairwise_tree<NW>(t);
+        for (int i = 0; i < 4; ++i) kr[4 * cc + i] = x[i];
+        if (KV8 && cc % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int v = 0; v < CV; ++v) {
+        const int j = (4 * (v / RPI) + g) * RPI + v % RPI, jc = min(j, np_max - 1);
+        float x[EW];
+        if constexpr (KV8) {
+          const float4 f = KvQ8(const_cast<float*>(v_cache), n_kv, max_seq, HD).load(kv_row + jc, HD, dim0 / 4);
+          if constexpr (EW == 4) {
+            x[0] = f.x; x[1] = f.y; x[2] = f.z; x[3] = f.w;
+          } else if constexpr (EW == 2) {
+            x[0] = dim0 & 2 ? f.z : f.x;
+            x[1] = dim0 & 2 ? f.w : f.y;
+          } else {
+            const float lo = dim0 & 1 ? f.y : f.x, hi = dim0 & 1 ? f.w : f.z;
+            x[0] = dim0 & 2 ? hi : lo;
+          }
+        } else {
+          const float* src = vc + (uint32_t)(jc * HD + dim0);
+          if constexpr (EW == 4) {
+            const f32x4 f = *(const f32x4*)src;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = f[e];
+          } else if constexpr (EW == 2) {
+            const float2 f = *(const float2*)src;
+            x[0] = f.x; x[1] = f.y;
+          } else {
+            x[0] = *src;
           }
         }
-      } else {
-        for (int idx = tid; idx < nt * 4 * HD; idx += NTA) {
-          const int u = idx / (4 * HD), r4 = idx % (4 * HD);
-          const int h = hg + r4 / HD;
-          if (h < G) {
-            const float* redu = red + u * NW * 4 * HD;
-            float t[NW];
 #pragma unroll
-            for (int w = 0; w < NW; ++w) t[w] = redu[w * 4 * HD + r4];
-            const size_t pbase = ((size_t)((sl + u) * n_kv + kvh) * n_chunks + c) * G;
-            PO[(pbase + h) * HD + (r4 % HD)] = pairwise_tree<NW>(t);
-          }
+        for (int e = 0; e < EW; ++e) vr[e][v] = x[e];
+        if (KV8 && v % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < NS; ++k) {
+        asm("" : "+v"(kr[k]));   // the loads stay unconditional
+        kr[k] = kin ? kr[k] : 0.0f;
+      }
+#pragma unroll
+      for (int cc = 0; cc < NS / 4; ++cc) transpose_groups(kr + 4 * cc);
+#pragma unroll
+      for (int v = 0; v < CV; ++v) {
+        const int j = (4 * (v / RPI) + g) * RPI + v % RPI;
+#pragma unroll
+        for (int e = 0; e < EW; ++e) {
+          asm("" : "+v"(vr[e][v]));
+          vr[e][v] = j < np_max ? vr[e][v] : 0.0f;
         }
       }
-      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (tid < nt * G) {
-      const int u = tid / G, h = tid % G;
-      const size_t pbase = ((size_t)((sl + u) * n_kv + kvh) * n_chunks + c) * G;
-      PML[(pbase + h) * 2] = ml[(u * G + h) * 2];
-      PML[(pbase + h) * 2 + 1] = ml[(u * G + h) * 2 + 1];
+    const int tl = ta + l16, np = min(C, pos0 + t0 + tl + 1 - p0);   // this lane's token and its rows
+    const bool live = tl < n && np > 0;
+    for (int h0 = 0; h0 < G; h0 += HB) {
+      const int nb = min(HB, G - h0);
+      const bool more = h0 + HB < G || ta + 16 < tend;
+      __syncthreads();   // q is there; everyone has read the last scores
+      for (int qt = qs; qt < nb; qt += QS) {
+        const float* qrow = sm_q + (HD == 128 ? (qt * 8 + (l16 >> 1)) * QP + (l16 & 1) * 4 : (qt * 16 + l16) * QP) + g;
+        f32x4 x = score_tree<NS>(kr, [&](int k) { return qrow[(HD == 128 ? 8 : 4) * k]; });
+        float m = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int v = 4 * p + r, j = (4 * (v / RPI) + g) * RPI + v % RPI;
+          x[r] = j < np ? x[r] * inv_sqrt : -INFINITY;
+          m = vmax_nonan(m, x[r]);
+        }
+        m = vmax_nonan(m, xor_lane<16>(m));
+        m = vmax_nonan(m, xor_lane<32>(m));
+        if (g == 0) sm_m[qt][p][l16] = m;
+        *(f32x4*)&sm_e[qt][l16 * 4 + g][4 * p] = x;
+      }
+      __syncthreads();
+      if (more) copy_q(h0 + HB < G ? ta : ta + 16, h0 + HB < G ? h0 + HB : 0);
+      for (int qt = qs; qt < nb; qt += QS) {   // this wave's scores become exponentials
+        float m = sm_m[qt][0][l16];
+#pragma unroll
+        for (int k = 1; k < NP; ++k) m = vmax_nonan(m, sm_m[qt][k][l16]);
+        f32x4 e = *(const f32x4*)&sm_e[qt][l16 * 4 + g][4 * p];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int v = 4 * p + r, j = (4 * (v / RPI) + g) * RPI + v % RPI;
+          const float ex = hx_exp(e[r] - m);
+          e[r] = j < np ? ex : 0.0f;
+        }
+        *(f32x4*)&sm_e[qt][l16 * 4 + g][4 * p] = e;
+      }
+      wait_q();
+      __syncthreads();
+      for (int qt = 0; qt < nb; ++qt) {
+        float e[CV];
+#pragma unroll
+        for (int k = 0; k < CV / 4; ++k) {
+          const f32x4 f = *(const f32x4*)&sm_e[qt][l16 * 4 + g][4 * k];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) e[4 * k + r] = f[r];
+        }
+        f32x4 o[EW];
+        pv_trees<EW, CV, RPI, NU>(vr, e, o);
+        const size_t pb = (((size_t)tl * n_kv + kvh) * n_chunks + c) * G + h0 + qt;
+        if (live) {
+          // register r of dim tile e: dim 16 EW wid + EW (4 g + r) + e, so a lane's
+          // 4 EW values are contiguous and the 4 lane groups fill whole lines (stored
+          // as 8-byte pieces 16 bytes apart, 2048 tokens took 743 us, not 662)
+          float* dst = PO + pb * HD + 16 * EW * wid + 4 * EW * g;
+#pragma unroll
+          for (int i = 0; i < EW; ++i) {
+            f32x4 f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) f[k] = o[(4 * i + k) % EW][(4 * i + k) / EW];
+            *(f32x4*)(dst + 4 * i) = f;
+          }
+        }
+        if (wid == qt) {   // (m, l): the 64-lane butterfly over the positions, e0 + e1 first at C = 128
+          float m = sm_m[qt][0][l16];
+#pragma unroll
+          for (int k = 1; k < NP; ++k) m = vmax_nonan(m, sm_m[qt][k][l16]);
+          float l;
+          auto over_groups = [&](float* t) {
+            float s = pairwise_tree<RPI>(t);
+            s = s + xor_lane<16>(s);
+            return s + xor_lane<32>(s);
+          };
+          if constexpr (C == 128) {
+            float t[RPI];
+#pragma unroll
+            for (int k = 0; k < RPI; ++k) t[k] = e[k] + e[RPI + k];
+            l = over_groups(t);
+          } else {
+            l = over_groups(e);
+            if constexpr (NU == 2) l = l + over_groups(e + RPI);
+          }
+          if (live && g == 0) *(float2*)(PML + pb * 2) = make_float2(m, l);
+        }
+      }
     }
   }
 }
@@ -1849,10 +1977,7 @@ int hh_prefill_attn_launch(int hd, const float* QB, const float* k_cache, const 
                            int max_seq, int pos0, int t0, int n, int n_chunks, float* PO, float* PML,
                            const float* gate, int gate_row, int kv_q8, int8_t* yq, float* yd, float* yf,
                            hipStream_t s) {
-  // tokens per split pass: 4 at head_dim 128, 1 at 256 (measured on the 8B and
-  // 9B/27B shapes; more tokens per pass cost occupancy at 256)
-  const int NTOK = hd == 128 ? 4 : 1;
-  const int G = n_heads / n_kv, TT = 16;
+  const int G = n_heads / n_kv;
   if (G > 8 || n_kv * G != n_heads || (hd != 128 && hd != 256)) return 1;
   const int cn = 8192 / hd;
   // token t (sequence length pos0 + t + 1) takes the wide chunk past seq_wide
@@ -1860,33 +1985,21 @@ int hh_prefill_attn_launch(int hd, const float* QB, const float* k_cache, const 
   const int tw = std::min(t0 + n, std::max(t0, seq_wide - pos0));
   auto pass = [&](int ta, int na, int C) -> int {
     if (na <= 0) return 0;
-    // the grid's chunk count: the caller's stride for the narrow pass (its XCD
-    // spread), for the wide one the chunks it reaches rounded up to 3 mod 8 the
-    // same way; workgroups past a token tile's last chunk exit
-    int nc = n_chunks;
-    if (C != cn) {
-      nc = (pos0 + ta + na + C - 1) / C;
-      nc += (3 - nc % 8 + 8) % 8;
-    }
-    const size_t split_lds = 4 * (NTOK * ((size_t)G * C + 2 * G + (ATTN_NT / 64) * 4 * (size_t)hd) + 8);
+    // the chunks that the pass reaches; workgroups past a token tile's last one exit
+    const int nc = (pos0 + ta + na + C - 1) / C;
     const size_t merge_lds = 4 * (4 * (size_t)n_chunks);
-    dim3 g1(nc, n_kv, (na + TT - 1) / TT), g2((na * n_heads + 3) / 4);
-#define HH_PSPLIT(HDV, KV, GM, GTV, CV)                                                                           \
-  hipLaunchKernelGGL((k_attn_prefill_split<HDV, ATTN_NT, KV, GM, HDV == 128 ? 4 : 1, GTV, CV>), g1, dim3(ATTN_NT), \
-                     split_lds, s, QB, k_cache, v_cache, n_heads, n_kv, max_seq, pos0, ta + na, ta, TT, n_chunks, PO, \
-                     PML)
-    // group sizes 4 and 8 get exact trip counts (GT), others read G at run time
-#define HH_PSPLIT_G(HDV, KV, CV)                                      \
-  do {                                                                \
-    if (G == 4) HH_PSPLIT(HDV, KV, 4, 4, CV);                         \
-    else if (G < 4) HH_PSPLIT(HDV, KV, 4, 0, CV);                     \
-    else if (G == 8) HH_PSPLIT(HDV, KV, 8, 8, CV);                    \
-    else HH_PSPLIT(HDV, KV, 8, 0, CV);                                \
-  } while (0)
+    // 64 tokens per workgroup, which share its K and V, unless that leaves CUs idle
+    int tpw = 4;
+    while (tpw > 1 && (long)nc * n_kv * ((na + 16 * tpw - 1) / (16 * tpw)) < 2048) tpw /= 2;
+    dim3 g1((unsigned)nc * n_kv * ((na + 16 * tpw - 1) / (16 * tpw))), g2((na * n_heads + 3) / 4);
+    // 4 waves hold a narrow chunk's K and V in registers, 8 a wide one's
+#define HH_PSPLIT(HDV, KV, NWV, CV)                                                                               \
+  hipLaunchKernelGGL((k_attn_prefill_split<HDV, KV, NWV, CV>), g1, dim3(64 * NWV), 0, s, QB, k_cache, v_cache,    \
+                     n_heads, n_kv, max_seq, pos0, ta, na, nc, tpw, n_chunks, PO, PML)
 #define HH_PSPLIT_C(HDV, KV)                                          \
   do {                                                                \
-    if (C == 8192 / HDV) HH_PSPLIT_G(HDV, KV, 8192 / HDV);            \
-    else HH_PSPLIT_G(HDV, KV, 16384 / HDV);                           \
+    if (C == 8192 / HDV) HH_PSPLIT(HDV, KV, 4, 8192 / HDV);           \
+    else HH_PSPLIT(HDV, KV, 8, 16384 / HDV);                          \
   } while (0)
     if (hd == 128) {
       if (kv_q8) HH_PSPLIT_C(128, true); else HH_PSPLIT_C(128, false);
@@ -1898,7 +2011,6 @@ int hh_prefill_attn_launch(int hd, const float* QB, const float* k_cache, const 
                          pos0, ta, na, gate, gate_row, yq, yd, yf);
     }
 #undef HH_PSPLIT_C
-#undef HH_PSPLIT_G
 #undef HH_PSPLIT
     return hipGetLastError() == hipSuccess ? 0 : 1;
   };

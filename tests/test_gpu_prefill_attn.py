@@ -69,6 +69,62 @@ def test_prefill_attention_modes_vs_float64(ctx, nh, nkv, hd, pos0, n):
         assert np.array_equal(one.cpu().numpy(), got[0][t].reshape(-1)), t
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0,n", [
+    (5, 1, 128, 0, 1), (7, 1, 256, 3, 17), (16, 8, 128, 15, 16),      # group sizes 5, 7, 2; one token, one tile
+    (8, 8, 128, 2040, 41), (24, 4, 256, 2031, 49),                    # narrow to wide chunks inside the prompt
+    (32, 8, 128, 63, 1100), (16, 4, 256, 0, 900)])                    # 16 to 64 tokens per workgroup
+def test_prefill_split_equals_decode_at_edges(ctx, nh, nkv, hd, pos0, n):
+    """The split pass on the matrix instructions restates the decode split bit for bit: the
+    rows at tile, chunk and width edges equal hh_attention's, with the cache's rows past
+    the prompt not numbers."""
+    rng = np.random.default_rng(nh * 100 + hd + pos0 + n)
+    ms = pos0 + n + 70
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    q = rng.standard_normal((n, nh, hd)).astype(np.float32)
+    k = rng.standard_normal((nkv, ms, hd)).astype(np.float32) * 2
+    v = rng.standard_normal((nkv, ms, hd)).astype(np.float32)
+    k[:, pos0 + n:] = np.nan
+    v[:, pos0 + n:] = np.nan
+    dk, dv = dev(k), dev(v)
+    out = torch.full((n * nh * hd + 64,), 7.0, dtype=torch.float32, device="cuda")
+    print(f"prefill split {nh}/{nkv} x {hd}, pos0 {pos0}, {n} tokens", flush=True)
+    ctx.attention_prefill(dev(q), dk, dv, nh, nkv, hd, ms, pos0, n, 0, out)
+    ctx.sync()
+    got = out.cpu().numpy()
+    assert (got[n * nh * hd:] == 7.0).all()
+    got = got[:n * nh * hd].reshape(n, -1)
+    edges = {0, 1, 15, 16, 17, 31, 32, 63, 64, n // 2, n - 2, n - 1}
+    edges |= {p - pos0 + d for p in (64, 128, 512, 1024, 2048) for d in (-2, -1, 0, 1)}   # chunks, the wide rule
+    one = torch.zeros(nh * hd, dtype=torch.float32, device="cuda")
+    for t in sorted(e for e in edges if 0 <= e < n):
+        ctx.attention(dev(q[t]), dk, dv, nh, nkv, hd, ms, pos0 + t + 1, one)
+        ctx.sync()
+        assert np.array_equal(one.cpu().numpy(), got[t]), t
+
+
+@pytest.mark.parametrize("hd,nkv", [(128, 8), (256, 4)])
+def test_prefill_split_q8_kv_equals_decode(ctx, hd, nkv):
+    """The same over a Q8_0 cache, where the prompt crosses into the wide chunks: the
+    logits after a batched prompt equal those after the prompt token by token."""
+    from hearth_amd import GGML_Q2_0, Model, ModelConfig
+    cfg = ModelConfig(d_model=1024, n_layers=1, n_heads=2 * nkv, n_kv_heads=nkv, head_dim=hd, d_ffn=1024, vocab=512,
+                      max_seq=2112, wtype=GGML_Q2_0, kv_type=8)
+    toks = np.random.default_rng(hd).integers(0, 512, 40).tolist()
+    got = []
+    for batched in (True, False):
+        m = Model(ctx, cfg)
+        m.synthesize(3)
+        m.prefill_kv_synthetic(4, 2030)
+        if batched:
+            m.prefill(toks[:-1], 2030)
+        else:
+            for i, t in enumerate(toks[:-1]):
+                m.forward(t, 2030 + i, want_logits=False)
+        got.append(m.forward(toks[-1], 2030 + len(toks) - 1)[0])
+        m.close()
+    assert np.array_equal(got[0], got[1])
+
+
 def _model_env(ctx, cfg, seed, env):
     from hearth_amd import Model
     old = os.environ.get("HH_PREFILL_ATTN")
