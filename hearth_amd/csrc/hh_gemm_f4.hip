@@ -275,7 +275,7 @@ HH_DEV void store_tile(float* __restrict__ out, const f32x16& v, int row0, int t
   }
 }
 
-// The product straight from the GGUF blocks, for few tokens: WR waves of 32 rows,
+// The product straight from the GGUF blocks: WR waves of 32 rows,
 // all on the same 32 tokens.  Per 128-column step the activation tile is copied to
 // LDS and the weight blocks are expanded there; two LDS buffers, the next step's
 // global loads in registers over the whole compute of the current one.
@@ -350,6 +350,92 @@ __global__ __launch_bounds__(64 * WR, 2) void k_gemm_f4(const uint8_t* __restric
     __syncthreads();
   }
   store_tile(out, sum, r0 + wid * 32, g * 32, n, seq, vec_out);
+}
+
+// The same for a grid too small to fill the CUs that way: one 32 x 32 tile per
+// workgroup of 8 waves.  A round takes 16 column blocks, two per wave: the wave loads
+// and expands its own weights and activations, and leaves its block accumulators in
+// LDS; after the barrier every lane adds its two outputs' 16 block products in block
+// order (sum += acc * dw, the scalar order).  So a short prompt still spreads a
+// matrix over all CUs, with one memory round trip per 2048 columns.
+template <int FMT>
+__global__ __launch_bounds__(512, 2) void k_gemm_f4s(const uint8_t* __restrict__ w,
+                                                     const uint8_t* __restrict__ tiles, float* __restrict__ out,
+                                                     int n, int K, int seq, int n_groups, int vec_out) {
+#pragma clang fp contract(off)
+  constexpr int NB = 16;
+  __shared__ __align__(16) float acc[NB][4][64][4];   // [block][output / 4][lane][output % 4]
+  __shared__ float dws[NB][32];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, l32 = lane & 31, lh = lane >> 5;
+  const int n_rt = (n + 31) / 32, r0 = blockIdx.x % n_rt * 32, g = blockIdx.x / n_rt;
+  const int nkb = K / 128, scale_b = lh ? 130 : 134;
+  const uint8_t* wrow = w + (size_t)min(r0 + l32, n - 1) * ((size_t)nkb * blk_bytes<FMT>());
+  const int q = wid >> 1, j0 = 2 * (wid & 1);   // this lane's outputs 4 q + j0, + 1
+  float s0 = 0.0f, s1 = 0.0f;
+  for (int base = 0; base < nkb; base += NB) {
+    const int nb = min(NB, nkb - base);
+    WRaw<FMT> R[2];
+    uint32_t sc[2];
+    u32x4 b16[2][4];
+    u32x2 b8[2][4];
+    f32x4 da[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {   // blocks past the end re-read the last (not added)
+      const int kb = min(base + 2 * wid + i, nkb - 1);
+      const uint8_t* blk = wrow + (size_t)kb * blk_bytes<FMT>();
+      w_load<FMT>(R[i], blk, lh);
+      sc[i] = *(const uint16_t*)(blk + scale_off<FMT>());
+      const uint8_t* at = tiles + ((size_t)kb * n_groups + g) * AT_BYTES;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int p = (s * 2 + lh) * 32 + l32;
+        b16[i][s] = *(const u32x4*)(at + p * 16);
+        b8[i][s] = *(const u32x2*)(at + AT_HI + p * 8);
+      }
+      da[i] = *(const f32x4*)(at + AT_D + l32 * 16);
+    }
+    if (base) __syncthreads();   // the last round's accumulators have been read
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      uint32_t o[8];
+      w_expand<FMT>(R[i], lh, o);
+      i32x8 a[4] = {};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {   // both halves' words to all lanes
+        const auto r = __builtin_amdgcn_permlane32_swap(o[k], o[k], false, false);
+        a[k >> 2][k & 3] = (int)r[0];
+        a[2 + (k >> 2)][k & 3] = (int)r[1];
+      }
+      f32x16 c[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) c[s] = sub_dots(a[s], op_fp6(b16[i][s], b8[i][s]), scale_b);
+      const int slot = 2 * wid + i;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        f32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = block_sum(c, 4 * k + j, da[i]);
+        *(f32x4*)acc[slot][k][lane] = v;
+      }
+      if (lh == 0) dws[slot][l32] = h2f(sc[i]);
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int k = 0; k < nb; ++k) {
+      const float2 v = *(const float2*)&acc[k][q][lane][j0], dw = *(const float2*)&dws[k][8 * q + 4 * lh + j0];
+      s0 += v.x * dw.x;
+      s1 += v.y * dw.y;
+    }
+  }
+  const int tok = g * 32 + l32, row = r0 + 8 * q + 4 * lh + j0;
+  if (tok >= seq) return;
+  float* o = out + (size_t)tok * n + row;
+  if (vec_out) {
+    if (row < n) *(float2*)o = make_float2(s0, s1);   // n % 4 == 0
+  } else {
+    if (row < n) o[0] = s0;
+    if (row + 1 < n) o[1] = s1;
+  }
 }
 
 // ---- expanded weights ----
@@ -560,12 +646,20 @@ int hh_act_tiles_launch(int fmt, const uint8_t* x, const int8_t* xq, const float
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-// Few tokens run straight from the GGUF blocks; from F4X_SEQ tokens on the weights
-// are expanded once per call (3 bytes of traffic per 4 weights), which takes their
-// expansion and their scattered loads out of every workgroup.  8B gate+up (24576 x
-// 4096), us direct / expanded: 128 tokens 51 / 68, 512 tokens 157 / 143, 2048 tokens
-// 573 / 515.
-constexpr int F4X_SEQ = 256;
+// Few tokens run straight from the GGUF blocks.
+// One tile per workgroup while two rounds of those at most cover the grid (2 per CU):
+// us with 128-row workgroups / so, Q2_0: 37 tokens through 4096 x 2048 16.3 / 8.0,
+// 5120 x 17408 at 16 tokens 102 / 37; 12288 x 2048 at 33 tokens (768 tiles) 16.5 / 15.2,
+// at 128 (1536) 21 / 28; 5120 x 5120 at 128 (640) 35 / 36.
+static bool single_tiles(int n, int ng) { return (long)((n + 31) / 32) * ng <= (ng <= 2 ? 768 : 512); }
+// Past that the weights are expanded once per call (3 bytes of traffic per 4 weights)
+// where enough tokens share them, which takes their expansion and their scattered loads
+// out of every workgroup: us direct / expanded, 24576 x 4096 Q2_0 at 128 tokens 50 / 58,
+// 200 87 / 88, 256 91 / 89, 512 157 / 130, 2048 573 / 435; 12288 x 4096 PTQ1_0 (whose
+// trits cost more) at 96 53 / 36.
+static bool expands(int fmt, int n, int seq) {
+  return seq >= (fmt == FMT_PT ? 96 : 224) && !single_tiles(n, (seq + 31) / 32);
+}
 constexpr size_t F4X_SLAB = (size_t)128 << 20;   // most bytes of expanded weights at a time
 
 static int slab_rows(int n, int K) {   // rows per expansion: whole 256-row tiles
@@ -573,8 +667,8 @@ static int slab_rows(int n, int K) {   // rows per expansion: whole 256-row tile
   return (int)std::min<size_t>((n + 255) / 256, std::max<size_t>(1, F4X_SLAB / per)) * 256;
 }
 
-size_t hh_gemm_f4_wbytes(int n, int K, int seq) {
-  return seq >= F4X_SEQ ? (size_t)(slab_rows(n, K) / 32) * (K / 128) * WT_BYTES : 0;
+size_t hh_gemm_f4_wbytes(int fmt, int n, int K, int seq) {
+  return expands(fmt, n, seq) ? (size_t)(slab_rows(n, K) / 32) * (K / 128) * WT_BYTES : 0;
 }
 
 int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* tiles, int seq, uint8_t* wtiles,
@@ -582,12 +676,17 @@ int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* ti
   if (K <= 0 || K % 128 != 0 || n <= 0 || seq <= 0 || (fmt != FMT_Q2 && fmt != FMT_Q1 && fmt != FMT_PT)) return 1;
   const int ng = (seq + 31) / 32, ngp = act_groups(seq);
   const int vec = n % 4 == 0 && ((uintptr_t)out & 15) == 0;
-  if (seq < F4X_SEQ || !wtiles) {
-    const dim3 grid((unsigned)((n + 127) / 128) * ng);
-#define HH_F4(F) hipLaunchKernelGGL((k_gemm_f4<F, 4>), grid, dim3(256), 0, s, w, tiles, out, n, K, seq, ngp, vec)
-    if (fmt == FMT_Q2) HH_F4(FMT_Q2);
-    else if (fmt == FMT_Q1) HH_F4(FMT_Q1);
-    else HH_F4(FMT_PT);
+  if (!expands(fmt, n, seq) || !wtiles) {
+    const bool small = single_tiles(n, ng);
+    const dim3 grid(small ? (unsigned)((n + 31) / 32) * ng : (unsigned)((n + 127) / 128) * ng);
+#define HH_F4(F)                                                                                                   \
+  if (small) hipLaunchKernelGGL((k_gemm_f4s<F>), grid, dim3(512), 0, s, w, tiles, out, n, K, seq, ngp, vec);        \
+  else hipLaunchKernelGGL((k_gemm_f4<F, 4>), grid, dim3(256), 0, s, w, tiles, out, n, K, seq, ngp, vec)
+    switch (fmt) {
+      case FMT_Q2: HH_F4(FMT_Q2); break;
+      case FMT_Q1: HH_F4(FMT_Q1); break;
+      default: HH_F4(FMT_PT); break;
+    }
 #undef HH_F4
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }

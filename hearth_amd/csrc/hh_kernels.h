@@ -150,9 +150,9 @@ constexpr int HH_ACT_TILE_BYTES = 6656;
 size_t hh_act_tiles_bytes(int K, int seq);
 int hh_act_tiles_launch(int fmt, const uint8_t* x, const int8_t* xq, const float* xd, int K, int seq, uint8_t* tiles,
                         hipStream_t s);
-// wtiles: hh_gemm_f4_wbytes(n, K, seq) bytes of scratch (null: not used, slower from
-// 256 tokens on)
-size_t hh_gemm_f4_wbytes(int n, int K, int seq);
+// wtiles: hh_gemm_f4_wbytes(fmt, n, K, seq) bytes of scratch for expanded weights (null:
+// not used, slower from some 200 tokens on)
+size_t hh_gemm_f4_wbytes(int fmt, int n, int K, int seq);
 int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* tiles, int seq, uint8_t* wtiles,
                       float* out, hipStream_t s);
 

@@ -556,8 +556,14 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   int n_in_max = 0;
   for (const Layer& L : m->layers) n_in_max = std::max(n_in_max, L.n_in);
   const int kmax = std::max(std::max(d, F), std::max(nq, vdim));
-  const size_t wt_max = std::max(std::max(hh_gemm_f4_wbytes(n_in_max, d, S), hh_gemm_f4_wbytes(2 * F, d, S)),
-                                 std::max(hh_gemm_f4_wbytes(d, F, S), hh_gemm_f4_wbytes(d, std::max(nq, vdim), S)));
+  size_t wt_max = 0;   // expanded weights of the largest projection that wants them
+  auto with = [&](int n, int K) { wt_max = std::max(wt_max, hh_gemm_f4_wbytes(m->wfmt, n, K, S)); };
+  for (const Layer& L : m->layers) {
+    with(L.n_in, d);
+    with(d, L.gdn ? vdim : nq);
+  }
+  with(2 * F, d);
+  with(d, F);
   // scratch layout
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align256(off + bytes); return o; };
@@ -852,7 +858,7 @@ int hh_gemm_q8(hh_ctx* c, int type, const void* w, int64_t n_rows, int64_t n_col
   // weights (1- and 2-bit formats), or int8 rows plus f32 block scales (Q8_0)
   const size_t nq = (size_t)seq_len * n_cols;
   const size_t act = align256(fmt == FMT_Q8 ? nq : hh_act_tiles_bytes((int)n_cols, (int)seq_len));
-  const size_t extra = fmt == FMT_Q8 ? nq / 32 * 4 : hh_gemm_f4_wbytes((int)n_rows, (int)n_cols, (int)seq_len);
+  const size_t extra = fmt == FMT_Q8 ? nq / 32 * 4 : hh_gemm_f4_wbytes(fmt, (int)n_rows, (int)n_cols, (int)seq_len);
   if (c->gemm_scratch_bytes < act + extra) {
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (c->gemm_scratch) HIP_TRY(hipFree(c->gemm_scratch));

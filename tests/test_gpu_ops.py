@@ -253,8 +253,9 @@ def test_gemm_bit_exact_vs_per_token_dot(ctx, oracle, t, n, k, seq):
 
 @pytest.mark.parametrize("t", [41, 42, 143])
 @pytest.mark.parametrize("n,k,seq", [
-    (1, 128, 1), (33, 256, 32), (127, 384, 33), (257, 640, 255),      # straight from the blocks
-    (31, 128, 256), (257, 256, 257), (130, 384, 300), (512, 1024, 511),  # expanded, 128 x 64 by 8 waves; 1..8 steps
+    (1, 128, 1), (33, 256, 32), (127, 2048, 33), (257, 2176, 255), (31, 4224, 65),   # one tile per workgroup
+    (24641, 256, 30), (12225, 384, 33), (8193, 128, 90),              # 128 rows per workgroup
+    (8200, 128, 224), (4097, 256, 257), (4226, 384, 300), (4096, 1024, 511),  # expanded, 128 x 64 by 8 waves; 1..8 steps
     (4096, 128, 1024), (4095, 256, 1000),                             # 128 x 64 by 4 waves
     (6144, 128, 2048), (4096, 384, 2048)])                            # 128 x 128 and 256 x 128
 def test_gemm_tiles_bit_exact(ctx, oracle, t, n, k, seq):
