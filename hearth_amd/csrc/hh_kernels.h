@@ -164,7 +164,7 @@ int hh_rope_launch(float* x, int n_heads, int hd, int rope_dim, const float* tab
                    hipStream_t s);
 int hh_embed_launch(int type, const uint8_t* table, int d, const StepState* st, float* hidden,
                     const float* signs, int had_block, hipStream_t s);
-int hh_argmax_launch(const float* logits, int64_t n, const int* counts, float pen, int rule,
+int hh_argmax_launch(const float* logits, int64_t n, const uint32_t* past, int64_t n_past, float pen, int rule,
                      float* part_val, int* part_idx, int* counter, uint32_t* out, hipStream_t s);
 int hh_count_tokens_launch(const uint32_t* past, int64_t n_past, int* counts, hipStream_t s);
 int hh_fill_i32_launch(int* p, int64_t n, int v, hipStream_t s);

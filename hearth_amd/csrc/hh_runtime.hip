@@ -91,8 +91,6 @@ struct hh_ctx {
   float* part_val = nullptr;
   int* part_idx = nullptr;
   int* counter = nullptr;
-  int* counts = nullptr;
-  int64_t counts_n = 0;
   hipEvent_t ev[8] = {};
   void* attn_scratch = nullptr;     // standalone attention partials + counters
   size_t attn_scratch_bytes = 0;
@@ -743,7 +741,6 @@ int hh_ctx_destroy(hh_ctx* c) {
   hipFree(c->part_val);
   hipFree(c->part_idx);
   hipFree(c->counter);
-  if (c->counts) hipFree(c->counts);
   if (c->attn_scratch) hipFree(c->attn_scratch);
   if (c->gemm_scratch) hipFree(c->gemm_scratch);
   for (hipEvent_t e : c->ev)
@@ -1028,18 +1025,8 @@ int hh_argmax(hh_ctx* c, const float* logits, int64_t n, const uint32_t* past, i
   if (!c || !logits || !out || (n_past && !past)) return fail(HH_ERR_INVALID, "null argument");
   if (n <= 0 || n > (1ll << 31) - 1) return fail(HH_ERR_DIM, "bad length");
   if (rule != 0 && rule != 1) return fail(HH_ERR_INVALID, "rule must be 0 or 1");
-  const int* counts = nullptr;
-  if (rule == 0 && n_past > 0) {
-    if (c->counts_n < n) {
-      if (c->counts) hipFree(c->counts);
-      HIP_TRY(hipMalloc(&c->counts, sizeof(int) * (size_t)n));
-      c->counts_n = n;
-    }
-    KTRY(hh_fill_i32_launch(c->counts, n, 0, c->stream));
-    KTRY(hh_count_tokens_launch(past, n_past, c->counts, c->stream));
-    counts = c->counts;
-  }
-  KTRY(hh_argmax_launch(logits, n, counts, pen, rule, c->part_val, c->part_idx, c->counter, out, c->stream));
+  KTRY(hh_argmax_launch(logits, n, past, std::max<int64_t>(n_past, 0), pen, rule, c->part_val, c->part_idx, c->counter,
+                        out, c->stream));
   return HH_OK;
 }
 

@@ -232,6 +232,32 @@ def test_argmax_rules(ctx, oracle):
     assert int(host(out)[0]) == want == 20
 
 
+@pytest.mark.parametrize("n", [1, 4095, 4096, 4097, 151936, 256 * 4096 + 5])
+def test_argmax_ranges(ctx, oracle, n):
+    """Workgroup ranges of 4096 logits and past one range per workgroup: the penalty's
+    counts and the tie rules over range edges, against the sampler and numpy; all
+    logits the type's lowest, and -inf."""
+    lib = oracle.load()
+    rng = np.random.default_rng(n)
+    out = torch.zeros(1, dtype=torch.int32, device="cuda")
+    x = rng.standard_normal(n).astype(np.float32)
+    top = np.unique(np.clip(np.array([0, 1, 4094, 4095, 4096, 4097, n // 2, n - 2, n - 1]), 0, n - 1))
+    x[top] = 6.0
+    for n_past in (1, 200, 3000):
+        past = np.concatenate([top, top[::2], rng.integers(0, n, n_past)])[:max(n_past, 1)].astype(np.uint32)
+        xc = x.copy()
+        want = lib.ho_sample_greedy_dense(xc.ctypes.data, n, past.ctypes.data, len(past), 1.1)
+        for _ in range(2):
+            ctx.argmax(dev(x), n, dev(past), len(past), 1.1, 0, out)
+            assert int(host(out)[0]) == want
+        ctx.argmax(dev(x), n, dev(past), len(past), 1.1, 1, out)   # rule 1 takes no penalty
+        assert int(host(out)[0]) == top[0]
+    for low in (np.finfo(np.float32).min, -np.inf):
+        for rule, want in ((0, n - 1), (1, 0)):
+            ctx.argmax(dev(np.full(n, low, np.float32)), n, None, 0, 1.0, rule, out)
+            assert int(host(out)[0]) == want
+
+
 @pytest.mark.parametrize("t", [41, 42, 8, 143])
 @pytest.mark.parametrize("n,k,seq", [(200, 512, 70), (2048, 2048, 16), (64, 5120, 1), (130, 1024, 129)])
 def test_gemm_bit_exact_vs_per_token_dot(ctx, oracle, t, n, k, seq):
