@@ -232,6 +232,36 @@ def test_argmax_rules(ctx, oracle):
     assert int(host(out)[0]) == want == 20
 
 
+@pytest.mark.parametrize("n", [1, 31, 1023, 1024, 1025, 2049, 4096, 4097, 8192, 8193, 17408])
+def test_norm_and_quantize_sizes(ctx, oracle, n):
+    """rms_norm at the row lengths where its register form ends (three rows, in place
+    too) against float64, and quantize_q8_0 of the same values bit for bit at any
+    length, from an address that is only 4-byte and to one that is only byte aligned."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((3, n)).astype(np.float32) * 3
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    x64 = x.astype(np.float64)
+    want = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-6) * w
+    dx, out = dev(x), torch.zeros(3 * n + 8, dtype=torch.float32, device="cuda")
+    ctx.rms_norm(dx, dev(w), 1e-6, 3, n, out)
+    ctx.rms_norm(dx, dev(w), 1e-6, 3, n, dx)
+    got = host(out)
+    assert np.all(got[3 * n:] == 0)
+    # the sum of squares: n / 256 + 10 roundings of at most 2^-24 each, halved by the root; 4 more after it
+    assert np.abs(got[:3 * n].reshape(3, n) / want - 1).max() <= (n / 512 + 9) * 2.0 ** -24
+    assert np.array_equal(host(dx).reshape(-1), got[:3 * n])
+    src = torch.zeros(3 * n + 1, dtype=torch.float32, device="cuda")
+    src[1:] = dev(x.reshape(-1))
+    nb = (3 * n + 31) // 32 * 34
+    q8 = torch.full((nb + 9,), 0xAB, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    ctx.quantize_q8_0(src.data_ptr() + 4, 3 * n, q8.data_ptr() + 1)
+    ctx.sync()
+    b = host(q8)
+    assert b[0] == 0xAB and np.all(b[1 + nb:] == 0xAB)
+    assert np.array_equal(b[1:1 + nb], oracle.quantize_q8_0(x.reshape(-1)))
+
+
 @pytest.mark.parametrize("n", [1, 4095, 4096, 4097, 151936, 256 * 4096 + 5])
 def test_argmax_ranges(ctx, oracle, n):
     """Workgroup ranges of 4096 logits and past one range per workgroup: the penalty's
