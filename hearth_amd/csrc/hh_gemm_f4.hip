@@ -701,17 +701,18 @@ int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* ti
     else HH_WT(FMT_PT);
 #undef HH_WT
     // The workgroup tile with the least time for this grid on 256 CUs, from the
-    // measured time of one 128-column step with a CU's workgroups resident (us):
-    //   256 x 128 (rows x tokens), 1 per CU : 2.13
-    //   128 x 128, 2 per CU : 2.2 (1.35 alone)
-    //   128 x 64, 2 per CU, 4 waves : 1.25 (0.9 alone); 8 waves, 1 per CU : 0.8
+    // measured time of one 128-column step with a CU's workgroups resident, their start
+    // and stores spread over 32 steps (us):
+    //   256 x 128 (rows x tokens), 1 per CU : 2.5
+    //   128 x 128, 2 per CU : 2.6 (1.35 alone)
+    //   128 x 64, 2 per CU, 4 waves : 1.33 (0.9 alone); 8 waves, 1 per CU : 0.8
     auto wgs = [&](int r, int t) { return (long)((nr + r - 1) / r) * ((ng + t - 1) / t); };
     auto rounds = [](long g, double pair, double alone) {
       const long full = g / 512, rest = g % 512;
       return full * pair + (rest == 0 ? 0.0 : rest <= 256 ? alone : pair);
     };
-    const double ta = ((wgs(256, 4) + 255) / 256) * 2.13, tb = rounds(wgs(128, 4), 2.2, 1.35);
-    const double tc = rounds(wgs(128, 2), 1.25, 0.9), td = ((wgs(128, 2) + 255) / 256) * 0.8;
+    const double ta = ((wgs(256, 4) + 255) / 256) * 2.5, tb = rounds(wgs(128, 4), 2.6, 1.35);
+    const double tc = rounds(wgs(128, 2), 1.33, 0.9), td = ((wgs(128, 2) + 255) / 256) * 0.8;
     const double best = std::min(std::min(ta, tb), std::min(tc, td));
 #define HH_F4X(RT, TT, WR, WT, NS)                                                                               \
   hipLaunchKernelGGL((k_gemm_f4x<RT, TT, WR, WT, NS>),                                                           \
