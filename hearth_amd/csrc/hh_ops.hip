@@ -1426,9 +1426,8 @@ __global__ __launch_bounds__(256) void k_attn_prefill_merge(const float* __restr
 // scores), so it matches the split/merge path (and token-by-token decode) to
 // fp32 rounding, not bit for bit; that path stays the default.
 //
-// Workgroup = W = G*T waves, T = max(1, 8 / G) token tiles of 16 (4 to 8
-// waves); wave w handles query head kvh*G + w % G for tokens s0 + 16 (w / G)
-// + 0..15, so a staged chunk serves up to 8 query rows per position.  The 1-D
+// Workgroup = 16 tokens x one kv head, G waves; wave w handles query head kvh*G + w,
+// so a staged chunk serves G query rows per position.  The 1-D
 // grid runs the kv heads fastest: with the round-robin dispatch over the 8
 // XCDs, one kv head's workgroups share an XCD and its L2 (n_kv dividing 8).
 // The workgroup stages each 32-position chunk of its kv head's K and V in LDS
@@ -1448,7 +1447,6 @@ __global__ __launch_bounds__(512) void k_attn_prefill_mfma(const float* __restri
                                                            const float* __restrict__ gate, int gate_row,
                                                            int8_t* __restrict__ yq, float* __restrict__ yd,
                                                            float* __restrict__ yf) {
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
   // chunk positions (64 measured the same at head_dim 128), LDS row stride,
   // dim blocks, 16-position tiles
   constexpr int CHK = 32, RS = HD + 4, NJ = HD / 16, NQT = CHK / 16;
@@ -1456,11 +1454,12 @@ __global__ __launch_bounds__(512) void k_attn_prefill_mfma(const float* __restri
   __shared__ __align__(16) float Vs[CHK * RS];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nth = blockDim.x;
   const int mi = lane & 15, g = lane >> 4;
-  const int G = n_heads / n_kv, T = G >= 8 ? 1 : 8 / G;
-  const int kvh = (int)blockIdx.x % n_kv, h = wid % G, qh = kvh * G + h;
-  const int tile0 = t0 + ((int)blockIdx.x / n_kv) * 16 * T;   // first token of the workgroup
-  const int last = min(t0 + n, tile0 + 16 * T) - 1;           // its last valid token
-  const int sq_raw = tile0 + 16 * (wid / G) + mi;
+  const int G = n_heads / n_kv;
+  const int kvh = (int)blockIdx.x % n_kv, qh = kvh * G + wid;
+  // first token of the workgroup; the last tokens, which see every chunk, first
+  const int tile0 = t0 + ((int)gridDim.x / n_kv - 1 - (int)blockIdx.x / n_kv) * 16;
+  const int last = min(t0 + n, tile0 + 16) - 1;               // its last valid token
+  const int sq_raw = tile0 + mi;
   const bool qvalid = sq_raw < t0 + n;
   const int sq = min(sq_raw, t0 + n - 1);                     // out-of-range lanes compute a valid row
   const int pq = pos0 + sq;
@@ -2088,8 +2087,11 @@ int hh_prefill_attn_mfma_launch(int hd, const float* QB, const float* k_cache, c
                                 int kv_q8, int8_t* yq, float* yd, float* yf, hipStream_t s) {
   const int G = n_heads / n_kv;
   if (G < 1 || G > 8 || n_kv * G != n_heads || n <= 0) return 1;
-  const int T = G >= 8 ? 1 : 8 / G;
-  dim3 grid(((n + 16 * T - 1) / (16 * T)) * n_kv), block(64 * G * T);
+  // one 16-token tile per workgroup, one wave per query head (8 / G tiles, so that 8
+  // waves shared a staged chunk, left CUs idle and gained nothing where they did not: a
+  // 9B layer, 16/4 heads x 256, 1024 tokens 313 -> 235 us; 8B, 32/8 x 128, 512 tokens
+  // 80 -> 55, 2048 tokens 439 -> 355)
+  dim3 grid(((n + 15) / 16) * n_kv), block(64 * G);
 #define HH_PMFMA(HDV, KV) \
   hipLaunchKernelGGL((k_attn_prefill_mfma<HDV, KV>), grid, block, 0, s, QB, k_cache, v_cache, n_heads, n_kv, max_seq, \
                      pos0, t0, n, gate, gate_row, yq, yd, yf)
