@@ -39,6 +39,26 @@ def _model(ctx, cfg, seed, chunked):
     return m
 
 
+def test_sequential_blocks_equal_decode(ctx):
+    """k_gdn_rec_rows at token counts around its 8-token blocks (its output waves run one
+    block behind): state and logits equal those of the tokens fed one at a time."""
+    cfg = CONFIGS["9b-hybrid-q2"].replace(n_layers=2, max_seq=256, vocab=1024)
+    m = _model(ctx, cfg, 29, False)
+    toks = np.random.default_rng(3).integers(0, 1024, 40).tolist()
+    for n in (1, 2, 7, 8, 9, 16, 17, 31):
+        got = []
+        for batched in (True, False):
+            m.reset()
+            if batched:
+                m.prefill(toks[:n], 0)
+            else:
+                for i in range(n):
+                    m.forward(toks[i], i, want_logits=False)
+            got.append((m.download_state(0), m.download_state(1), m.forward(toks[n], n)[0]))
+        assert all(np.array_equal(a, b) for a, b in zip(*got)), n
+    m.close()
+
+
 @pytest.mark.parametrize("n_prompt,split", [(300, 0), (130, 67), (40, 0)], ids=["300", "130-in-two-calls", "40"])
 def test_chunked_prefill_matches_sequential(ctx, oracle, n_prompt, split):
     prompt = [oracle.synth_token(5, i, 248320) for i in range(n_prompt)]
