@@ -133,8 +133,10 @@ PEAK_INT8_TOPS = 5000.0
 
 def prefill_leg(m, cfg, n_tok: int) -> dict:
     """forward_batch of an n_tok seeded prompt at positions 0.. (overwrites the
-    synthetic KV; runs after the decode measurement).  The layer GEMMs run on
-    int8 MFMA; attention and the row kernels on the vector units."""
+    synthetic KV; runs after the decode measurement).  The layer GEMMs
+    (FP4 x FP6 operands, exact integer block dots) and the attention run on MFMA,
+    the row kernels on the vector units.  The matrix fraction is stated against the
+    int8 dense peak."""
     rng = np.random.default_rng(7)
     toks = rng.integers(0, cfg.vocab, n_tok).tolist()
     m.prefill(toks[:64], 0)                       # warm-up (scratch, code)

@@ -498,15 +498,13 @@ int enqueue_step(hh_model* m, hipStream_t s, int only_layer, unsigned stages) {
 
 
 
-// Batched prefill of a dense model (forward_batch, mod.rs:899-1221): tokens
-// toks[0..S) at positions pos0.. through every layer with the int8-MFMA GEMM
-// and row kernels that restate the decode step's arithmetic, writing the KV
-// cache; no logits (mod.rs:1201-1218 computes only the last token's, which the
-// caller runs through the decode step).
 // Batched prefill (forward_batch, mod.rs:899-1221) of S prompt tokens from
-// pos0: every projection is one MFMA GEMM over the S token rows.  Dense and
-// qwen35 full-attention layers run the split/merge attention per 128-token
-// tile; GDN layers run the per-token prep in parallel and the recurrence in
+// pos0, writing the KV cache; no logits (mod.rs:1201-1218 computes only the
+// last token's, which the caller runs through the decode step).  Every
+// projection is one MFMA GEMM over the S token rows; the row kernels restate
+// the decode step's arithmetic.  Dense and qwen35 full-attention layers run
+// the split/merge attention over as many tokens as the split partials' bytes
+// allow; GDN layers run the per-token prep in parallel and the recurrence in
 // token order per v-head (the state stays in registers).  The result is the
 // state that feeding the tokens one at a time leaves, bit for bit.
 #ifndef PF_ATTN_BYTES

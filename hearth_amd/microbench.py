@@ -10,7 +10,7 @@ as such) are reported beside the HBM figures.
     python -m hearth_amd.microbench [--reps 1000] [--json]
     python -m hearth_amd.microbench --copy-mb 512    (plain device copy of known
         size: the calibration run for rocprofv3 FETCH_SIZE / WRITE_SIZE counters)
-    python -m hearth_amd.microbench --prefill        (batched int8-MFMA GEMM at the
+    python -m hearth_amd.microbench --prefill        (batched MFMA GEMM at the
         27B and 8B FFN shapes, 2048 tokens, against the dense int8 MFMA peak)
 """
 import argparse

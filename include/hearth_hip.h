@@ -98,8 +98,9 @@ int hh_gemv_q8(hh_ctx* ctx, int ggml_type, const void* w, int64_t n_rows, int64_
 /* Batched quantized GEMM for prefill: out[s*n_rows + r] = dot_fn(w + r*row_bytes,
  * x_q8 + s*(n_cols/32)*34, n_cols) for every token s < seq_len.  Replaces
  * ThreadPool::par_dot_rows_batched with DotFn / DotFn2 (pool.rs:40-80, :568-618;
- * matmul.rs:580-674 matmul_batch).  Runs on int8 MFMA; each output is bit-identical
- * to hh_gemv_q8 on that token, as the reference's paired kernels are to its
+ * matmul.rs:580-674 matmul_batch).  Runs on MFMA (FP4 x FP6 for the 1- and 2-bit
+ * formats, int8 for Q8_0; both give the exact integer block dots); each output is
+ * bit-identical to hh_gemv_q8 on that token, as the reference's paired kernels are to its
  * single-token dot (q2_0.rs:936-986).  x_q8: seq_len rows of n_cols/32 standard
  * Q8_0 blocks.  n_cols: a positive multiple of 128. */
 int hh_gemm_q8(hh_ctx* ctx, int ggml_type, const void* w, int64_t n_rows, int64_t n_cols,
@@ -227,8 +228,8 @@ int hh_model_generate(hh_model* m, const uint32_t* prompt, int n_prompt, int sta
                       float repeat_pen, uint32_t* out_tokens, float* last_logits_host);
 
 /* Batched prefill (LlamaModel::forward_batch, mod.rs:899-1221): runs
- * tokens[0..n) at positions start_pos.. through every layer with the int8-MFMA
- * GEMM (hh_gemm_q8) and writes their K/V; computes no logits (the reference
+ * tokens[0..n) at positions start_pos.. through every layer with the MFMA GEMM
+ * (hh_gemm_q8) and writes their K/V; computes no logits (the reference
  * computes only the last token's, mod.rs:1201-1218: feed that token to
  * hh_model_forward).  On qwen35 hybrids the GDN layers run their per-token
  * prep in parallel and the recurrence in token order; the reference has no
