@@ -560,19 +560,21 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   }
   with(2 * F, d);
   with(d, F);
-  // scratch layout
+  // scratch layout; a GEMM's operands (activation tiles, expanded weights) and the
+  // attention's partials are never live together, so they share one region
+  const size_t po = align256((size_t)TA * c.n_kv_heads * n_chunks * G * hd * 4);
+  const size_t pml = (size_t)TA * c.n_kv_heads * n_chunks * G * 2 * 4;
+  const size_t act = align256(hh_act_tiles_bytes(kmax, S));
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align256(off + bytes); return o; };
   const size_t oH = take((size_t)S * d * 4), oXq = take((size_t)S * kmax), oXd = take((size_t)S * (kmax / 32) * 4),
                oQKV = take((size_t)S * n_in_max * 4), oQB = take((size_t)S * nq * 4),
                oT = take((size_t)S * d * 4), oGU = take((size_t)S * 2 * F * 4),
-               oPO = take((size_t)TA * c.n_kv_heads * n_chunks * G * hd * 4),
-               oPML = take((size_t)TA * c.n_kv_heads * n_chunks * G * 2 * 4),
+               oPart = take(std::max(po + pml, act + wt_max)),
                oGQK = take(hyb ? (size_t)S * 2 * kdim * 4 : 0), oGV = take(hyb ? (size_t)S * vdim * 4 : 0),
                oGAB = take(hyb ? (size_t)S * 2 * c.ssm_n_v_heads * 4 : 0),
                oGDEC = take(hyb ? (size_t)S * c.ssm_n_v_heads * 4 : 0), oGO = take(hyb ? (size_t)S * vdim * 4 : 0),
                oRot = take(c.had_block > 0 ? (size_t)S * std::max(std::max(vdim, nq), F) * 4 : 0),
-               oAct = take(hh_act_tiles_bytes(kmax, S)), oWt = take(wt_max),
                oChunk = take(hyb && chunked ? hh_gdn_chunk_scratch_bytes(c.ssm_n_v_heads, S) : 0);
   if (off > m->pf_cap) {
     if (m->pf_buf) HIP_TRY(hipFree(m->pf_buf));
@@ -585,13 +587,13 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   float* H = (float*)(B + oH);
   int8_t* Xq = (int8_t*)(B + oXq);
   float* Xd = (float*)(B + oXd);
-  uint8_t* Act = B + oAct;
+  uint8_t* Act = B + oPart;
   float* QKV = (float*)(B + oQKV);
   float* QB = (float*)(B + oQB);
   float* T = (float*)(B + oT);
   float* GU = (float*)(B + oGU);
-  float* PO = (float*)(B + oPO);
-  float* PML = (float*)(B + oPML);
+  float* PO = (float*)(B + oPart);
+  float* PML = (float*)(B + oPart + po);
   // Hadamard fold (qwen35.rs:881-970): every matmul input row is rotated
   // before Q8_0; producers write f32 rows to Rot, k_rot_q8_rows quantizes them
   const bool had = c.had_block > 0;
@@ -603,7 +605,7 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   };
   auto gemm = [&](const uint8_t* w, int n, int K, float* out) -> int {
     const int rc = hh_act_tiles_launch(m->wfmt, nullptr, Xq, Xd, K, S, Act, s);
-    return rc ? rc : hh_gemm_f4_launch(m->wfmt, w, n, K, Act, S, wt_max ? B + oWt : nullptr, out, s);
+    return rc ? rc : hh_gemm_f4_launch(m->wfmt, w, n, K, Act, S, wt_max ? Act + act : nullptr, out, s);
   };
   KTRY(hh_embed_rows_launch(c.head_type, m->token_embd->d, d, toks, S, H, latent ? signs_of(m, d) : nullptr,
                             latent ? c.had_block : 0, s));
