@@ -1605,77 +1605,97 @@ HH_DEV bool better(int rule, float v2, int i2, float v1, int i1) {
   return rule == 0 ? (v2 > v1 || (v2 == v1 && i2 > i1)) : (v2 > v1 || (v2 == v1 && i2 < i1));
 }
 
-// One workgroup per 4096 logits: the ranges' past tokens are counted in LDS (each
-// workgroup reads the whole list), so a call is one launch and needs no count table.
-// The last workgroup to finish reduces the partials.  Q8_0 head of 151936 x 4096 and
-// the choice with 200 past tokens: 130.3 us with a fill, a count and 594 workgroups
-// contending for the counter, 123.6 so (the GEMV is 112 of it).
-constexpr int ARG_NT = 1024, ARG_PER = 4, ARG_RANGE = ARG_NT * ARG_PER, ARG_MAX_WG = 256;
-HH_DEV void argmax_reduce(int rule, float& bv, int& bi, float* sv, int* si) {   // all lanes end with the best
+// One workgroup per NT PER logits: the ranges' past tokens are counted in LDS (each
+// workgroup reads the whole list, eight ids per lane in flight), so a call is one
+// launch and needs no count table.  The last workgroup to finish reduces the
+// partials, one wave of each workgroup taking part: every wave that crosses a device
+// fence writes its cache back, and 16 of them in the last workgroup took 8 us (4096
+// logits 14.0 us a call so, 4.6 with one wave, 6.5 as 16 workgroups of 4 waves with
+// a count table).
+constexpr int ARG_MAX_WG = 256;
+HH_DEV void argmax_wave(int rule, float& bv, int& bi) {   // all lanes end with the best
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const float v = __shfl_xor(bv, o, 64);
     const int i = __shfl_xor(bi, o, 64);
     if (better(rule, v, i, bv, bi)) { bv = v; bi = i; }
   }
-  if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
-  __syncthreads();
-  for (int w = 0; w < ARG_NT / 64; ++w)
-    if (better(rule, sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
 }
-__global__ __launch_bounds__(ARG_NT) void k_argmax(const float* __restrict__ logits, int64_t n,
-                                                   const uint32_t* __restrict__ past, int64_t n_past, float pen,
-                                                   int rule, float* part_val, int* part_idx, int* counter,
-                                                   uint32_t* out) {
-  __shared__ int cnt[ARG_RANGE];
-  __shared__ float sv[ARG_NT / 64];
-  __shared__ int si[ARG_NT / 64];
-  __shared__ int is_last;
-  const int tid = threadIdx.x;
+template <int NT, int PER>
+__global__ __launch_bounds__(NT) void k_argmax(const float* __restrict__ logits, int64_t n,
+                                               const uint32_t* __restrict__ past, int64_t n_past, float pen,
+                                               int rule, float* part_val, int* part_idx, int* counter,
+                                               uint32_t* out) {
+  constexpr int RANGE = NT * PER, NW = NT / 64, IDS = 8;
+  __shared__ int cnt[RANGE];
+  __shared__ float sv[NW];
+  __shared__ int si[NW];
+  const int tid = threadIdx.x, lane = tid & 63;
   const bool do_pen = rule == 0 && n_past > 0 && !(fabsf(pen - 1.0f) < 1e-6f);
+  const int none = rule == 0 ? -1 : 0x7fffffff;
   float bv = -INFINITY;
-  int bi = rule == 0 ? -1 : 0x7fffffff;
-  for (int64_t base = (int64_t)blockIdx.x * ARG_RANGE; base < n; base += (int64_t)gridDim.x * ARG_RANGE) {
-    float v[ARG_PER];
+  int bi = none;
+  for (int64_t base = (int64_t)blockIdx.x * RANGE; base < n; base += (int64_t)gridDim.x * RANGE) {
+    float v[PER];
 #pragma unroll
-    for (int k = 0; k < ARG_PER; ++k) {
-      const int64_t i = base + tid + ARG_NT * k;
+    for (int k = 0; k < PER; ++k) {
+      const int64_t i = base + tid + NT * k;
       v[k] = logits[i < n ? i : n - 1];
     }
     if (do_pen) {
       __syncthreads();   // the last range's counts have been read
 #pragma unroll
-      for (int k = 0; k < ARG_PER; ++k) cnt[tid + ARG_NT * k] = 0;
+      for (int k = 0; k < PER; ++k) cnt[tid + NT * k] = 0;
       __syncthreads();
-      for (int64_t j = tid; j < n_past; j += ARG_NT) {
-        const int64_t r = (int64_t)past[j] - base;
-        if (r >= 0 && r < ARG_RANGE) atomicAdd(&cnt[r], 1);
+      const uint32_t b32 = (uint32_t)base;
+      int64_t j = 0;
+      for (; j + IDS * NT <= n_past; j += IDS * NT) {
+        uint32_t r[IDS];
+#pragma unroll
+        for (int u = 0; u < IDS; ++u) r[u] = past[j + tid + NT * u] - b32;
+#pragma unroll
+        for (int u = 0; u < IDS; ++u)
+          if (r[u] < (uint32_t)RANGE) atomicAdd(&cnt[r[u]], 1);
+      }
+      for (j += tid; j < n_past; j += NT) {
+        const uint32_t r = past[j] - b32;
+        if (r < (uint32_t)RANGE) atomicAdd(&cnt[r], 1);
       }
       __syncthreads();
     }
 #pragma unroll
-    for (int k = 0; k < ARG_PER; ++k) {
-      const int64_t i = base + tid + ARG_NT * k;
+    for (int k = 0; k < PER; ++k) {
+      const int64_t i = base + tid + NT * k;
       float x = v[k];
       if (do_pen)
-        for (int c = cnt[tid + ARG_NT * k]; c > 0; --c) x = (x > 0.0f) ? x / pen : x * pen;
+        for (int c = cnt[tid + NT * k]; c > 0; --c) x = (x > 0.0f) ? x / pen : x * pen;
       if (i < n && x == x && better(rule, x, (int)i, bv, bi)) { bv = x; bi = (int)i; }
     }
   }
-  argmax_reduce(rule, bv, bi, sv, si);
-  if (tid == 0) {
-    part_val[blockIdx.x] = bv;
-    part_idx[blockIdx.x] = bi;
-    __threadfence();
-    is_last = atomicAdd(counter, 1) == (int)gridDim.x - 1;
-  }
+  argmax_wave(rule, bv, bi);
+  if (lane == 0) { sv[tid >> 6] = bv; si[tid >> 6] = bi; }
   __syncthreads();
-  if (!is_last) return;
-  __threadfence();
-  bv = -INFINITY; bi = rule == 0 ? -1 : 0x7fffffff;
-  if (tid < (int)gridDim.x) { bv = part_val[tid]; bi = part_idx[tid]; }   // at most ARG_MAX_WG
-  argmax_reduce(rule, bv, bi, sv, si);
-  if (tid == 0) {
+  if (tid >= 64) return;
+  bv = lane < NW ? sv[lane] : -INFINITY;
+  bi = lane < NW ? si[lane] : none;
+  argmax_wave(rule, bv, bi);
+  if (gridDim.x > 1) {
+    int last = 0;
+    if (lane == 0) {
+      part_val[blockIdx.x] = bv;
+      part_idx[blockIdx.x] = bi;
+      __threadfence();
+      last = atomicAdd(counter, 1) == (int)gridDim.x - 1;
+    }
+    if (!__builtin_amdgcn_readfirstlane(last)) return;
+    __threadfence();
+    bv = -INFINITY;
+    bi = none;
+    for (int b = lane; b < (int)gridDim.x; b += 64)
+      if (better(rule, part_val[b], part_idx[b], bv, bi)) { bv = part_val[b]; bi = part_idx[b]; }
+    argmax_wave(rule, bv, bi);
+  }
+  if (lane == 0) {
     *out = (uint32_t)(bi < 0 ? 0 : bi);
     *counter = 0;
   }
@@ -1917,9 +1937,19 @@ int hh_attn_launch(const AttnArgs& a, hipStream_t s) {
 
 int hh_argmax_launch(const float* logits, int64_t n, const uint32_t* past, int64_t n_past, float pen, int rule,
                      float* part_val, int* part_idx, int* counter, uint32_t* out, hipStream_t s) {
-  const int nb = (int)std::min<int64_t>(ARG_MAX_WG, (n + ARG_RANGE - 1) / ARG_RANGE);
-  hipLaunchKernelGGL(k_argmax, dim3(nb), dim3(ARG_NT), 0, s, logits, n, past, n_past, pen, rule, part_val, part_idx,
-                     counter, out);
+  // Logits per lane: 4, so that a vocabulary fills the chip; 16 from 2^20 on, where 4
+  // leave several ranges, each with its own pass over the list, to a workgroup (2^24
+  // logits, 32768 past tokens: 61 us with 4, 39 with 16, 75 with a count table in
+  // memory); 1 where the list is the longer work, which more workgroups then share
+  // (4096 logits, 131072 past tokens: 31.8 with 4, 18.5 with 1, 22.0 with the table;
+  // 8192 tokens: 8.1 with 4).
+#define HH_ARGMAX(PER)                                                                                            \
+  hipLaunchKernelGGL((k_argmax<1024, PER>), dim3((unsigned)std::min<int64_t>(ARG_MAX_WG, (n + 1024 * PER - 1) / (1024 * PER))), \
+                     dim3(1024), 0, s, logits, n, past, n_past, pen, rule, part_val, part_idx, counter, out)
+  if (n >= (1 << 20)) HH_ARGMAX(16);
+  else if (n_past > 8192 && n <= 65536) HH_ARGMAX(1);
+  else HH_ARGMAX(4);
+#undef HH_ARGMAX
   return ok();
 }
 

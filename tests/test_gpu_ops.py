@@ -288,6 +288,28 @@ def test_argmax_ranges(ctx, oracle, n):
             assert int(host(out)[0]) == want
 
 
+@pytest.mark.parametrize("n,n_past", [(1, 8200), (1023, 8193), (1025, 20000), (65536, 8193), (65537, 8193),
+                                      (4096, 8191), (4096, 8192), (2 ** 20 - 1, 16385), (2 ** 20, 16383),
+                                      (256 * 16384 + 5, 9000)])
+def test_argmax_long_past(ctx, oracle, n, n_past):
+    """Past lists around whole blocks of eight ids per lane, and the range sizes that a
+    long list and a large vocabulary take: equal to the sampler's choice."""
+    lib = oracle.load()
+    rng = np.random.default_rng(n + n_past)
+    x = rng.standard_normal(n).astype(np.float32)
+    top = np.unique(np.clip(np.array([0, 1023, 1024, n // 2, n - 1]), 0, n - 1))
+    x[top] = 6.0
+    past = rng.integers(0, n, n_past).astype(np.uint32)
+    past[[0, n_past // 2, n_past - 1]] = [top[0], top[-1], top[len(top) // 2]]
+    out = torch.zeros(1, dtype=torch.int32, device="cuda")
+    xc = x.copy()
+    want = lib.ho_sample_greedy_dense(xc.ctypes.data, n, past.ctypes.data, n_past, 1.001)
+    print(f"argmax n={n} past={n_past}", flush=True)
+    for _ in range(2):
+        ctx.argmax(dev(x), n, dev(past), n_past, 1.001, 0, out)
+        assert int(host(out)[0]) == want
+
+
 @pytest.mark.parametrize("t", [41, 42, 8, 143])
 @pytest.mark.parametrize("n,k,seq", [(200, 512, 70), (2048, 2048, 16), (64, 5120, 1), (130, 1024, 129)])
 def test_gemm_bit_exact_vs_per_token_dot(ctx, oracle, t, n, k, seq):
