@@ -1426,9 +1426,9 @@ __global__ __launch_bounds__(256) void k_attn_prefill_merge(const float* __restr
 // scores), so it matches the split/merge path (and token-by-token decode) to
 // fp32 rounding, not bit for bit; that path stays the default.
 //
-// Workgroup = 16 tokens x one kv head, G waves; wave w handles query head kvh*G + w,
-// so a staged chunk serves G query rows per position.  The 1-D
-// grid runs the kv heads fastest: with the round-robin dispatch over the 8
+// Workgroup = T tiles of 16 tokens x one kv head, G*T waves (T = max(1, 4 / G)); wave w
+// handles query head kvh*G + w % G for tile w / G, so a staged chunk serves 4 to 8
+// query rows per position.  The 1-D grid runs the kv heads fastest: with the round-robin dispatch over the 8
 // XCDs, one kv head's workgroups share an XCD and its L2 (n_kv dividing 8).
 // The workgroup stages each 32-position chunk of its kv head's K and V in LDS
 // (dequantized when the cache holds Q8_0 rows).  Per chunk and wave:
@@ -1440,7 +1440,7 @@ __global__ __launch_bounds__(256) void k_attn_prefill_merge(const float* __restr
 //     in step r as position 4g + r of the lane's group, with A = V[4g + r][dim].
 // Then O / L, the qwen35 sigmoid gate, and the Q8_0 row of attn_output's input
 // in the GEMM's split layout (or the f32 row for a folded model).
-template <int HD, bool KV8>
+template <int HD, bool KV8, bool MANY>
 __global__ __launch_bounds__(512) void k_attn_prefill_mfma(const float* __restrict__ QB, const float* __restrict__ k_cache,
                                                            const float* __restrict__ v_cache, int n_heads, int n_kv,
                                                            int max_seq, int pos0, int t0, int n,
@@ -1454,11 +1454,12 @@ __global__ __launch_bounds__(512) void k_attn_prefill_mfma(const float* __restri
   __shared__ __align__(16) float Vs[CHK * RS];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nth = blockDim.x;
   const int mi = lane & 15, g = lane >> 4;
-  const int G = n_heads / n_kv;
-  const int kvh = (int)blockIdx.x % n_kv, qh = kvh * G + wid;
+  const int G = n_heads / n_kv, T = MANY ? nth / (64 * G) : 1, tw = MANY ? wid / G : 0;
+  const int kvh = (int)blockIdx.x % n_kv, qh = kvh * G + (MANY ? wid % G : wid);
   // first token of the workgroup; the last tokens, which see every chunk, first
-  const int tile0 = t0 + ((int)gridDim.x / n_kv - 1 - (int)blockIdx.x / n_kv) * 16;
-  const int last = min(t0 + n, tile0 + 16) - 1;               // its last valid token
+  const int wg0 = t0 + ((int)gridDim.x / n_kv - 1 - (int)blockIdx.x / n_kv) * 16 * T;
+  const int last = min(t0 + n, wg0 + 16 * T) - 1;             // its last valid token
+  const int tile0 = wg0 + 16 * tw;                            // this wave's first
   const int sq_raw = tile0 + mi;
   const bool qvalid = sq_raw < t0 + n;
   const int sq = min(sq_raw, t0 + n - 1);                     // out-of-range lanes compute a valid row
@@ -1500,6 +1501,7 @@ __global__ __launch_bounds__(512) void k_attn_prefill_mfma(const float* __restri
       *(float4*)(Vs + r * RS + 4 * cc) = vv;
     }
     __syncthreads();
+    if (MANY && pbase > pos0 + tile0 + 15) continue;   // past this wave's tokens (wave-uniform)
     // S^T for the chunk's 16-position tiles
     f32x4 sc[NQT];
 #pragma unroll
@@ -2117,14 +2119,22 @@ int hh_prefill_attn_mfma_launch(int hd, const float* QB, const float* k_cache, c
                                 int kv_q8, int8_t* yq, float* yd, float* yf, hipStream_t s) {
   const int G = n_heads / n_kv;
   if (G < 1 || G > 8 || n_kv * G != n_heads || n <= 0) return 1;
-  // one 16-token tile per workgroup, one wave per query head (8 / G tiles, so that 8
-  // waves shared a staged chunk, left CUs idle and gained nothing where they did not: a
-  // 9B layer, 16/4 heads x 256, 1024 tokens 313 -> 235 us; 8B, 32/8 x 128, 512 tokens
-  // 80 -> 55, 2048 tokens 439 -> 355)
-  dim3 grid(((n + 15) / 16) * n_kv), block(64 * G);
-#define HH_PMFMA(HDV, KV) \
-  hipLaunchKernelGGL((k_attn_prefill_mfma<HDV, KV>), grid, block, 0, s, QB, k_cache, v_cache, n_heads, n_kv, max_seq, \
-                     pos0, t0, n, gate, gate_row, yq, yd, yf)
+  // One wave per query head and 16-token tile, at least 4 waves per workgroup, which share
+  // the staged chunks.  Measured with 1, 2, 4 and 8 waves' worth of tiles over 2 to 2048
+  // tokens at positions 0, 300 and 1500: 4 waves were the fastest at every size for 1 and
+  // 2 query heads per kv head, and more than one tile never gained from 3 on.  us with
+  // 1 / 2 / 4 / 8 tiles, 2048 tokens: 16/16 heads x 128 424 / 326 / 245 / 316, 16/8 x 128
+  // 318 / 244 / 319 / 323, 24/8 x 128 327 / 400 / .., 32/8 x 128 345 / 403 / .., 16/4 x
+  // 256 467 / 611 / ...  (past 8 waves the count is what 8 hold)
+  const int T = std::max(1, 4 / G);
+  dim3 grid(((n + 16 * T - 1) / (16 * T)) * n_kv), block(64 * G * T);
+#define HH_PMFMA_T(HDV, KV, MANY)                                                                                      \
+  hipLaunchKernelGGL((k_attn_prefill_mfma<HDV, KV, MANY>), grid, block, 0, s, QB, k_cache, v_cache, n_heads, n_kv,     \
+                     max_seq, pos0, t0, n, gate, gate_row, yq, yd, yf)
+#define HH_PMFMA(HDV, KV)                                                \
+  do {                                                                   \
+    if (T > 1) HH_PMFMA_T(HDV, KV, true); else HH_PMFMA_T(HDV, KV, false); \
+  } while (0)
   if (hd == 128) {
     if (kv_q8) HH_PMFMA(128, true); else HH_PMFMA(128, false);
   } else if (hd == 256) {
@@ -2133,6 +2143,7 @@ int hh_prefill_attn_mfma_launch(int hd, const float* QB, const float* k_cache, c
     return 1;
   }
 #undef HH_PMFMA
+#undef HH_PMFMA_T
   return ok();
 }
 

@@ -10,7 +10,7 @@ restatement of causal softmax attention:
     float64 (its sums are regrouped, so this is its parity bar).
 
 Geometries cover head_dim 128 and 256, query groups 1, 3, 4, 6 and 8 (so the
-MFMA kernel's 1-4 token tiles per workgroup), partial 16-token tiles, a
+MFMA kernel's 4 tiles and 1 tile per workgroup), partial 16-token tiles, a
 prompt that starts past position 0 and one long enough for many chunks.  A
 model-level check runs a 9B-shaped slice and an 8B-shaped slice through the
 batched prefill both ways."""
@@ -100,6 +100,35 @@ def test_prefill_split_equals_decode_at_edges(ctx, nh, nkv, hd, pos0, n):
         ctx.attention(dev(q[t]), dk, dv, nh, nkv, hd, ms, pos0 + t + 1, one)
         ctx.sync()
         assert np.array_equal(one.cpu().numpy(), got[t]), t
+
+
+@pytest.mark.parametrize("nh,nkv,hd,pos0,n", [(16, 8, 128, 7, 49), (8, 8, 128, 0, 65), (2, 2, 256, 90, 63),
+                                              (8, 4, 256, 31, 17), (9, 3, 128, 12, 33)])
+def test_prefill_mfma_tiles_of_a_workgroup(ctx, nh, nkv, hd, pos0, n):
+    """The matrix form with several 16-token tiles per workgroup (1 and 2 query heads per
+    kv head) and one (3): a tile's rows equal, bit for bit, those of a call on that tile
+    alone."""
+    rng = np.random.default_rng(nh * 10 + hd + pos0 + n)
+    ms = pos0 + n + 5
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    q = rng.standard_normal((n, nh, hd)).astype(np.float32)
+    dk = dev(rng.standard_normal((nkv, ms, hd)).astype(np.float32) * 2)
+    dv = dev(rng.standard_normal((nkv, ms, hd)).astype(np.float32))
+    out = torch.full((n * nh * hd + 64,), 7.0, dtype=torch.float32, device="cuda")
+    print(f"prefill mfma tiles {nh}/{nkv} x {hd}, pos0 {pos0}, {n} tokens", flush=True)
+    ctx.attention_prefill(dev(q), dk, dv, nh, nkv, hd, ms, pos0, n, 1, out)
+    ctx.sync()
+    got = out.cpu().numpy()
+    assert (got[n * nh * hd:] == 7.0).all()
+    got = got[:n * nh * hd].reshape(n, -1)
+    for t in range(0, n, 16):
+        m = min(16, n - t)
+        one = torch.zeros(m * nh * hd, dtype=torch.float32, device="cuda")
+        ctx.attention_prefill(dev(q[t:t + m]), dk, dv, nh, nkv, hd, ms, pos0 + t, m, 1, one)
+        ctx.sync()
+        assert np.array_equal(one.cpu().numpy().reshape(m, -1), got[t:t + m]), t
+    want = _ref(q, dk.cpu().numpy(), dv.cpu().numpy(), pos0)
+    assert np.abs(got - want.reshape(n, -1)).max() / np.abs(want).max() < 1e-5
 
 
 @pytest.mark.parametrize("hd,nkv", [(128, 8), (256, 4)])
