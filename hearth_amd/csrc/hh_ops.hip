@@ -224,9 +224,45 @@ HH_DEV float4 slice_rope(float4 x, float4 sn, float4 cs, int c4, int rope_dim) {
 // the all-lanes butterfly x_l + x_(l^O) at that level, so the result for
 // value k is the butterfly sum with offsets LPR/2, ..., 1.  On return lane l
 // holds value k = (l % LPR) >> log2(LPR / NV).
-// At the offsets below 16 the lanes whose offset bit is set keep the upper half,
-// chosen per lane; the permlane swaps of 16 and 32 pair registers k and k + N/2
-// across the lanes themselves.
+// Lanes hand over their values in a lane-dependent register order: register
+// r of lane l holds value r ^ rs_perm<NV, LPR / 2>(l).  At each level below
+// offset 16 every lane then keeps registers [0, N/2) and sends [N/2, N): a
+// lane whose offset bit is set holds the upper half in the lower registers,
+// and its partner's upper registers hold that same half, so each kept sum is
+// the same pair of values, added in the same order, with no per-lane select.
+// (The permlane swaps of the offsets 16 and 32 pair registers r and r + N/2
+// across the lanes themselves.)
+template <int N, int O> HH_DEV int rs_perm(int lane) {
+  if constexpr (N > 1) return ((O < 16 && (lane & O)) ? N / 2 : 0) ^ rs_perm<N / 2, O / 2>(lane);
+  else return 0;
+}
+template <int N, int O> struct ReduceScatter {
+  static HH_DEV float run(float* v) {
+    if constexpr (N > 1) {
+      static_assert(O > 0, "more values than lanes");
+#pragma unroll
+      for (int k = 0; k < N / 2; ++k) {
+        if constexpr (O >= 16) v[k] = swap_pair_sum<O>(v[k], v[k + N / 2]);
+        else v[k] = v[k] + xor_lane<O>(v[k + N / 2]);
+      }
+      return ReduceScatter<N / 2, O / 2>::run(v);
+    } else {
+      float x = v[0];
+      if constexpr (O >= 32) x += xor_lane<32>(x);
+      if constexpr (O >= 16) x += xor_lane<16>(x);
+      if constexpr (O >= 8) x += xor_lane<8>(x);
+      if constexpr (O >= 4) x += xor_lane<4>(x);
+      if constexpr (O >= 2) x += xor_lane<2>(x);
+      if constexpr (O >= 1) x += xor_lane<1>(x);
+      return x;
+    }
+  }
+};
+
+// The same butterfly sum with values in the natural register order: lanes
+// whose offset bit is set keep the upper half, chosen per lane.  The decode
+// split uses it: its one pass is latency-bound, and the permuted order's
+// extra K addressing and q swaps cost more there than the selects.
 template <int N, int O> struct ReduceScatterSel {
   static HH_DEV float run(float* v, int lane) {
     if constexpr (N > 1) {
@@ -1318,6 +1354,209 @@ __global__ __launch_bounds__(64 * NWV, 2) void k_attn_prefill_split(const float*
   }
 }
 
+// The same for a few tokens (vec_tokens), where most of a 16-token tile would be empty:
+// workgroup (chunk c, kv head) holds K/V rows of chunk c in registers exactly as
+// k_attn_split does and runs the decode arithmetic (scores, chunk softmax, P.V and
+// their reduction order) on the vector unit once per token whose position reaches the
+// chunk, NTOK tokens per pass.  GMAX bounds the query heads per kv head (registers).
+template <int HD, int NTA, bool KV8, int GMAX, int NTOK, int GT, int C>
+__global__ __launch_bounds__(NTA) void k_attn_prefill_vec(const float* __restrict__ QB, const float* __restrict__ k_cache,
+                                                          const float* __restrict__ v_cache, int n_heads, int n_kv,
+                                                          int max_seq, int pos0, int t0, int n, int n_chunks,
+                                                          float* __restrict__ PO, float* __restrict__ PML) {
+  constexpr int LPR = HD / 4, RPI = NTA / LPR, NR = C / RPI, NW = NTA / 64;
+  extern __shared__ __align__(16) float sm[];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int c = blockIdx.x, kvh = blockIdx.y, G = GT > 0 ? GT : n_heads / n_kv;
+  const int p0 = c * C;
+  const int np_max = min(C, pos0 + t0 + n - p0);
+  if (np_max <= 0) return;
+  const int sub = tid / LPR, cc = tid % LPR;
+  float* sc = sm;                          // NTOK * G * C
+  float* ml = sc + NTOK * G * C;           // NTOK * 2 * G (+pad)
+  float* red = ml + ((NTOK * 2 * G + 4 + 3) & ~3);   // NTOK * NW waves * 4 heads * HD (16-byte aligned)
+  const size_t hstride = (size_t)max_seq * HD;
+  const float* kg = k_cache + (size_t)kvh * hstride + 4 * cc;
+  const float* vg = v_cache + (size_t)kvh * hstride + 4 * cc;
+  // K rows and q heads in the reduce-scatter's register order
+  // (ReduceScatter): K register i holds row (i ^ pi) * RPI + sub, q register
+  // h of a group of four head (h ^ ph); V rows stay in order (the P.V chain
+  // runs over i).  The q rows arrive normalized and rotated, so no step here
+  // needs the lanes of a row on one head.
+  constexpr int NV = 4 * NR;
+  const int rsp = rs_perm<NV, LPR / 2>(lane), pi = rsp % NR, ph = rsp / NR;
+  float4 kr[NR], vr[NR];
+  // every K row before the V rows (the scores need only K)
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int jk = (i ^ pi) * RPI + sub;
+    kr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (KV8) {
+      const size_t r = (size_t)kvh * max_seq + p0;
+      if (jk < np_max) kr[i] = KvQ8(const_cast<float*>(k_cache), n_kv, max_seq, HD).load(r + jk, HD, cc);
+    } else {
+      if (jk < np_max) kr[i] = *(const float4*)(kg + (size_t)(p0 + jk) * HD);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int j = i * RPI + sub;
+    vr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (KV8) {
+      const size_t r = (size_t)kvh * max_seq + p0;
+      if (j < np_max) vr[i] = KvQ8(const_cast<float*>(v_cache), n_kv, max_seq, HD).load(r + j, HD, cc);
+    } else {
+      if (j < np_max) vr[i] = *(const float4*)(vg + (size_t)(p0 + j) * HD);
+    }
+  }
+  const float inv_sqrt = 1.0f / sqrtf((float)HD);
+  constexpr int KSH = (LPR == 64 ? 6 : 5) - (NV == 32 ? 5 : NV == 16 ? 4 : 3);
+  // NTOK tokens per pass (each with the decode arithmetic of one token): their
+  // softmax rows spread over all waves and they share the barriers.  Tokens
+  // before the first whose position reaches the chunk skip it.
+  const int sl_first = max(0, p0 - pos0 - t0);
+  for (int sl = sl_first; sl < n; sl += NTOK) {
+    const int nt = min(NTOK, n - sl);
+#pragma unroll
+    for (int u = 0; u < NTOK; ++u) {
+      if (u >= nt) break;   // uniform
+      const int s = t0 + sl + u, np = min(C, pos0 + s + 1 - p0);
+      float4 q4[GMAX];
+#pragma unroll
+      for (int h = 0; h < GMAX; ++h) {
+        q4[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if ((h & ~3) < G) {
+          const int hs = (h & ~3) | ((h & 3) ^ ph);
+          const float* qp = QB + (size_t)s * n_heads * HD + (size_t)(kvh * G + hs) * HD + 4 * cc;
+          q4[h] = *(const float4*)(hs < G ? qp : attn_zero_row);
+        }
+      }
+      float* scu = sc + u * G * C;
+#pragma unroll
+      for (int hg = 0; hg < GMAX; hg += 4) {
+        if (hg >= G) break;
+        float v[NV];
+#pragma unroll
+        for (int hh = 0; hh < 4; ++hh) {
+          const float4 qq = hg + hh < GMAX ? q4[hg + hh] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+          for (int i = 0; i < NR; ++i) {
+            float pp = qq.x * kr[i].x;
+            pp = fmaf(qq.y, kr[i].y, pp);
+            pp = fmaf(qq.z, kr[i].z, pp);
+            pp = fmaf(qq.w, kr[i].w, pp);
+            v[hh * NR + i] = pp;
+          }
+        }
+        const float r = ReduceScatter<NV, LPR / 2>::run(v);
+        const int k = (lane & (LPR - 1)) >> KSH;
+        const int h = hg + k / NR, j = (k % NR) * RPI + sub;
+        if (h < G && (lane & ((1 << KSH) - 1)) == 0) scu[h * C + j] = (j < np) ? r * inv_sqrt : -INFINITY;
+      }
+    }
+    __syncthreads();
+    for (int pr = wid; pr < nt * G; pr += NW) {
+      const int u = pr / G, h = pr % G;
+      const int np = min(C, pos0 + t0 + sl + u + 1 - p0);
+      float* row = sc + (u * G + h) * C;
+      if constexpr (C <= 64) {
+        float x = lane < C ? row[lane] : -INFINITY;
+        float m = wave_max_nonan(x);
+        float e = (lane < np) ? hx_exp(x - m) : 0.0f;
+        float l = wave_sum(e);
+        if (lane < C) row[lane] = e;
+        if (lane == 0) { ml[(u * G + h) * 2] = m; ml[(u * G + h) * 2 + 1] = l; }
+      } else {   // C = 128, as the decode split
+        const float x0 = row[lane], x1 = row[64 + lane];
+        const float m = wave_max_nonan(fmaxf(x0, x1));
+        const float e0 = (lane < np) ? hx_exp(x0 - m) : 0.0f;
+        const float e1 = (64 + lane < np) ? hx_exp(x1 - m) : 0.0f;
+        const float l = wave_sum(e0 + e1);
+        row[lane] = e0;
+        row[64 + lane] = e1;
+        if (lane == 0) { ml[(u * G + h) * 2] = m; ml[(u * G + h) * 2 + 1] = l; }
+      }
+    }
+    __syncthreads();
+    for (int hg = 0; hg < G; hg += 4) {
+#pragma unroll
+      for (int u = 0; u < NTOK; ++u) {
+        if (u >= nt) break;
+        float acc[16];
+#pragma unroll
+        for (int hh = 0; hh < 4; ++hh) {
+          float o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
+          if (hg + hh < G) {
+            const float* eh = sc + (u * G + hg + hh) * C + sub;
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+              const float e = eh[i * RPI];
+              o0 = fmaf(e, vr[i].x, o0);
+              o1 = fmaf(e, vr[i].y, o1);
+              o2 = fmaf(e, vr[i].z, o2);
+              o3 = fmaf(e, vr[i].w, o3);
+            }
+          }
+          acc[hh * 4 + 0] = o0; acc[hh * 4 + 1] = o1; acc[hh * 4 + 2] = o2; acc[hh * 4 + 3] = o3;
+        }
+        float* redu = red + u * NW * 4 * HD;
+        if constexpr (LPR == 32) {
+          const bool up = (lane & 32) != 0;
+          float xs[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) xs[k] = swap_pair_sum<32>(acc[k], acc[k + 8]);
+#pragma unroll
+          for (int g = 0; g < 2; ++g)   // two 16-byte writes per lane, as the decode split
+            *(float4*)(redu + (wid * 4 + g + (up ? 2 : 0)) * HD + 4 * cc) =
+                make_float4(xs[4 * g], xs[4 * g + 1], xs[4 * g + 2], xs[4 * g + 3]);
+        } else {
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *(float4*)(redu + (wid * 4 + g) * HD + 4 * cc) =
+                make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
+        }
+      }
+      __syncthreads();
+      if constexpr (4 * HD == NTA) {
+        // lane tid owns value r4 = tid of every token u: its partial sits at
+        // a fixed offset from token u's block, one token stride apart
+        const int h = hg + tid / HD;
+        if (h < G) {
+          const size_t tok = (size_t)n_kv * n_chunks * G * HD;
+          float* dst = PO + (((size_t)sl * n_kv + kvh) * n_chunks + c) * G * HD + (size_t)hg * HD + tid;
+          for (int u = 0; u < nt; ++u) {
+            const float* redu = red + u * NW * 4 * HD;
+            float t[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) t[w] = redu[w * 4 * HD + tid];
+            dst[u * tok] = pairwise_tree<NW>(t);
+          }
+        }
+      } else {
+        for (int idx = tid; idx < nt * 4 * HD; idx += NTA) {
+          const int u = idx / (4 * HD), r4 = idx % (4 * HD);
+          const int h = hg + r4 / HD;
+          if (h < G) {
+            const float* redu = red + u * NW * 4 * HD;
+            float t[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) t[w] = redu[w * 4 * HD + r4];
+            const size_t pbase = ((size_t)((sl + u) * n_kv + kvh) * n_chunks + c) * G;
+            PO[(pbase + h) * HD + (r4 % HD)] = pairwise_tree<NW>(t);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (tid < nt * G) {
+      const int u = tid / G, h = tid % G;
+      const size_t pbase = ((size_t)((sl + u) * n_kv + kvh) * n_chunks + c) * G;
+      PML[(pbase + h) * 2] = ml[(u * G + h) * 2];
+      PML[(pbase + h) * 2 + 1] = ml[(u * G + h) * 2 + 1];
+    }
+  }
+}
+
 // Prefill attention, merge pass: k_attn_merge's arithmetic for token t0 + sl,
 // one wave per (token, query head): pair blockIdx.x * 4 + wave = sl * n_heads
 // + qh.  Lane l holds columns CPL*l .. CPL*l + CPL-1 (CPL = HD / 64) and runs
@@ -2063,6 +2302,21 @@ int hh_prefill_qk_launch(int hd, const float* QKV, int n_in, int n_heads, int n_
   return ok();
 }
 
+// Tokens of a split pass up to which k_attn_prefill_vec is the faster one: it takes about
+// 1 us (hd 128) to 2-3 us (hd 256, one token at a time) per token, the matrix form the
+// same for 1 to 16, growing with the query heads G per kv head.  us at position 0, vector /
+// matrix, split and merge: 32/8 heads x 128, 2 tokens 8.3 / 16.0, 8 14.5 / 15.5; 16/8 x 128,
+// 4 10.4 / 11.8, 5 12.1 / 11.8; 8/8 x 128, 3 9.4 / 9.9, 4 10.1 / 10.0; 16/4 x 256, 6 15.7 /
+// 17.0, 7 17.4 / 16.8; 24/4 x 256, 4 19.1 / 20.8, 5 22.4 / 20.9.  The line moves where the
+// chunks fill the CUs, since the matrix form's loads then weigh more: 8 tokens, 16/4 x 256 at
+// 7000 (440 chunks) 48.9 / 56.5; 32/8 x 128 at 1500 (192) 18.5 / 17.9.
+static int vec_tokens(int hd, int G, int workgroups) {
+  if (hd == 128) return std::min(8, G + (G > 2 ? 3 : 2) + (G == 4 && workgroups <= 64));
+  const int few = G == 8 ? 7 : G == 4 ? 6 : 4;   // 4 and 8 have exact trip counts
+  if (G <= 2) return few + (workgroups > 256 ? 2 : 0);
+  return few + (workgroups > 160) + (G == 4 && workgroups > 256);
+}
+
 // Attention for tokens [t0, t0 + n) of a prefill; PO/PML hold n tokens'
 // partials at a stride of n_chunks narrow chunks.  Each token uses the chunk
 // width the decode step uses at its sequence length (attn_chunk_for): the
@@ -2086,10 +2340,25 @@ int hh_prefill_attn_launch(int hd, const float* QB, const float* k_cache, const 
     int tpw = 4;
     while (tpw > 1 && (long)nc * n_kv * ((na + 16 * tpw - 1) / (16 * tpw)) < 2048) tpw /= 2;
     dim3 g1((unsigned)nc * n_kv * ((na + 16 * tpw - 1) / (16 * tpw))), g2((na * n_heads + 3) / 4);
+    const bool vec = na <= vec_tokens(hd, G, nc * n_kv);
+    // workgroup ids x + grid.x * y, grid.x = 3 mod 8: each kv head's chunk x on a different
+    // XCD of the round-robin dispatch; NTOK 4 at head_dim 128, 1 at 256 (occupancy)
+    const dim3 gv(nc + (3 - nc % 8 + 8) % 8, n_kv);
+    const size_t vec_lds = 4 * ((hd == 128 ? 4 : 1) * ((size_t)G * C + 2 * G + (ATTN_NT / 64) * 4 * (size_t)hd) + 8);
+#define HH_PVEC(HDV, KV, GM, GTV, CV)                                                                             \
+  hipLaunchKernelGGL((k_attn_prefill_vec<HDV, ATTN_NT, KV, GM, HDV == 128 ? 4 : 1, GTV, CV>), gv, dim3(ATTN_NT),  \
+                     vec_lds, s, QB, k_cache, v_cache, n_heads, n_kv, max_seq, pos0, ta, na, n_chunks, PO, PML)
     // 4 waves hold a narrow chunk's K and V in registers, 8 a wide one's
 #define HH_PSPLIT(HDV, KV, NWV, CV)                                                                               \
-  hipLaunchKernelGGL((k_attn_prefill_split<HDV, KV, NWV, CV>), g1, dim3(64 * NWV), 0, s, QB, k_cache, v_cache,    \
-                     n_heads, n_kv, max_seq, pos0, ta, na, nc, tpw, n_chunks, PO, PML)
+  do {                                                                                                            \
+    if (!vec)                                                                                                     \
+      hipLaunchKernelGGL((k_attn_prefill_split<HDV, KV, NWV, CV>), g1, dim3(64 * NWV), 0, s, QB, k_cache,         \
+                         v_cache, n_heads, n_kv, max_seq, pos0, ta, na, nc, tpw, n_chunks, PO, PML);              \
+    else if (G == 4) HH_PVEC(HDV, KV, 4, 4, CV);                                                                  \
+    else if (G < 4) HH_PVEC(HDV, KV, 4, 0, CV);                                                                   \
+    else if (G == 8) HH_PVEC(HDV, KV, 8, 8, CV);                                                                  \
+    else HH_PVEC(HDV, KV, 8, 0, CV);                                                                              \
+  } while (0)
 #define HH_PSPLIT_C(HDV, KV)                                          \
   do {                                                                \
     if (C == 8192 / HDV) HH_PSPLIT(HDV, KV, 4, 8192 / HDV);           \
@@ -2106,6 +2375,7 @@ int hh_prefill_attn_launch(int hd, const float* QB, const float* k_cache, const 
     }
 #undef HH_PSPLIT_C
 #undef HH_PSPLIT
+#undef HH_PVEC
     return hipGetLastError() == hipSuccess ? 0 : 1;
   };
   if (pass(t0, tw - t0, cn)) return 1;

@@ -154,6 +154,66 @@ def test_prefill_split_q8_kv_equals_decode(ctx, hd, nkv):
     assert np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("nh,nkv,hd,pos0", [
+    (8, 8, 128, 62), (16, 8, 128, 2045), (24, 8, 128, 0), (32, 8, 128, 2043), (10, 2, 128, 500), (16, 2, 128, 8189),
+    (4, 4, 256, 30), (8, 4, 256, 2046), (12, 4, 256, 3), (16, 4, 256, 2044), (24, 4, 256, 100), (16, 2, 256, 31),
+    (8, 8, 256, 4200)])
+def test_prefill_few_tokens_equal_decode(ctx, nh, nkv, hd, pos0):
+    """1 to 10 tokens, on both sides of every line between the vector pass and the matrix
+    form and across the narrow and wide chunks: each row equals hh_attention's bit for
+    bit, with the cache's rows past the prompt not numbers."""
+    rng = np.random.default_rng(nh * 100 + hd + pos0)
+    top = 10
+    ms = pos0 + top + 64
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    q = rng.standard_normal((top, nh, hd)).astype(np.float32)
+    k = rng.standard_normal((nkv, ms, hd)).astype(np.float32) * 2
+    v = rng.standard_normal((nkv, ms, hd)).astype(np.float32)
+    dq, dk, dv = dev(q), dev(k), dev(v)
+    print(f"prefill few tokens {nh}/{nkv} x {hd}, pos0 {pos0}", flush=True)
+    want = []
+    for t in range(top):
+        one = torch.zeros(nh * hd, dtype=torch.float32, device="cuda")
+        ctx.attention(dq[t].contiguous(), dk, dv, nh, nkv, hd, ms, pos0 + t + 1, one)
+        ctx.sync()
+        want.append(one.cpu().numpy())
+    for n in range(top, 0, -1):
+        dk[:, pos0 + n:] = float("nan")
+        dv[:, pos0 + n:] = float("nan")
+        out = torch.full((n * nh * hd + 64,), 7.0, dtype=torch.float32, device="cuda")
+        ctx.attention_prefill(dq, dk, dv, nh, nkv, hd, ms, pos0, n, 0, out)
+        ctx.sync()
+        got = out.cpu().numpy()
+        assert (got[n * nh * hd:] == 7.0).all()
+        for t in range(n):
+            assert np.array_equal(got[t * nh * hd:(t + 1) * nh * hd], want[t]), (n, t)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(16, 8, 128), (32, 8, 128), (16, 4, 256), (24, 4, 256)])
+def test_prefill_few_tokens_q8_kv_equals_decode(ctx, nh, nkv, hd):
+    """The same over a Q8_0 cache, through the batched prompt of a model: 3 tokens (the
+    vector pass) and 12 (the matrix form) from a position where the chunks turn wide."""
+    from hearth_amd import GGML_Q2_0, Model, ModelConfig
+    cfg = ModelConfig(d_model=1024, n_layers=1, n_heads=nh, n_kv_heads=nkv, head_dim=hd, d_ffn=1024, vocab=512,
+                      max_seq=2112, wtype=GGML_Q2_0, kv_type=8)
+    m = Model(ctx, cfg)
+    m.synthesize(3)
+    for pos0 in (9, 2046):
+        for n in (4, 13):
+            toks = np.random.default_rng(n).integers(0, 512, n).tolist()
+            got = []
+            for batched in (True, False):
+                m.prefill_kv_synthetic(4, pos0)
+                if batched:
+                    m.prefill(toks[:-1], pos0)
+                else:
+                    for i, t in enumerate(toks[:-1]):
+                        m.forward(t, pos0 + i, want_logits=False)
+                got.append(m.forward(toks[-1], pos0 + n - 1)[0])
+            assert np.array_equal(got[0], got[1]), (pos0, n)
+    m.close()
+
+
 def _model_env(ctx, cfg, seed, env):
     from hearth_amd import Model
     old = os.environ.get("HH_PREFILL_ATTN")
