@@ -40,6 +40,16 @@ def test_version_and_error_channel_without_gpu():
     assert cfg_rc == 1
 
 
+def test_operator_pointers():
+    """Raw addresses pass through as they are; None is a null pointer; a host tensor
+    gives its own address without a device being asked."""
+    import torch
+    from hearth_amd.lib import _ptrs
+    x = torch.zeros(4)
+    assert tuple(_ptrs(1 << 40, 2, 3)) == (1 << 40, 2, 3)
+    assert tuple(_ptrs(x, None, 7, x)) == (x.data_ptr(), 0, 7, x.data_ptr())
+
+
 def test_no_oracle_in_product():
     """The product package never imports or loads the oracle."""
     pkg = os.path.join(ROOT, "hearth_amd")
