@@ -21,7 +21,7 @@
 //
 // What bounds it: the combine, 6 VALU operations per output and 128-weight block (the
 // int8 form took 9); the matrix pipe is busy about a third as long.  8B gate+up
-// (24576 x 4096, Q2_0) over 2048 tokens: int8 form 795 us, here 443 us, of which the
+// (24576 x 4096, Q2_0) over 2048 tokens: int8 form 791 us, here 417 us, of which the
 // combine alone would take 0.25 ms.
 #include "hh_kernels.h"
 
@@ -646,29 +646,88 @@ int hh_act_tiles_launch(int fmt, const uint8_t* x, const int8_t* xq, const float
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-// Few tokens run straight from the GGUF blocks.
-// One tile per workgroup while two rounds of those at most cover the grid (2 per CU):
-// us with 128-row workgroups / so, Q2_0: 37 tokens through 4096 x 2048 16.3 / 8.0,
-// 5120 x 17408 at 16 tokens 102 / 37; 12288 x 2048 at 33 tokens (768 tiles) 16.5 / 15.2,
-// at 128 (1536) 21 / 28; 5120 x 5120 at 128 (640) 35 / 36.
-static bool single_tiles(int n, int ng) { return (long)((n + 31) / 32) * ng <= (ng <= 2 ? 768 : 512); }
-// Past that the weights are expanded once per call (3 bytes of traffic per 4 weights)
-// where enough tokens share them, which takes their expansion and their scattered loads
-// out of every workgroup: us direct / expanded, 24576 x 4096 Q2_0 at 128 tokens 50 / 58,
-// 200 87 / 88, 256 91 / 89, 512 157 / 130, 2048 573 / 435; 12288 x 4096 PTQ1_0 (whose
-// trits cost more) at 96 53 / 36.
-static bool expands(int fmt, int n, int seq) {
-  return seq >= (fmt == FMT_PT ? 96 : 224) && !single_tiles(n, (seq + 31) / 32);
-}
-constexpr size_t F4X_SLAB = (size_t)128 << 20;   // most bytes of expanded weights at a time
+// The forms of a product and the time each takes, from which the launcher chooses.
+// A form costs a start, and for each of its rounds (the workgroups that fit the 256
+// CUs at once) a fixed part and a part per 128 columns.  The figures are fits to 2829
+// measured products (K 128 .. 17408, 1024 .. 34816 rows, 2 .. 2048 tokens, the three
+// formats, weights cold), where the choice by them takes 0.1% longer than the fastest
+// form on average and, from K = 1024, 10% at most.  (Thresholds on the tokens and the
+// grid alone, set at K = 4096, took up to 57% longer, and at K = 1024 longer than an int8
+// MFMA kernel: Q2_0, 6144 x 1024, 224 tokens 13.2 us expanded in 128 x 64 tiles, 12.3
+// int8, 10.4 straight from the blocks, the form chosen here.  Of the products from K =
+// 1024 int8 keeps one corner, PTQ1_0 12288 x 1024 at 96 and 128 tokens: 14.3, here 15.6.)
+enum : int { F4_TILE, F4_ROWS, X_128x64_8, X_128x64_4, X_128x128, X_256x128, N_FORMS };
+constexpr int FORM_ROWS[N_FORMS] = {32, 128, 128, 128, 128, 256};
+constexpr int FORM_GROUPS[N_FORMS] = {1, 1, 2, 2, 4, 4};   // 32-token groups
 
+// us of one pass over n rows in a form (the expanded ones without their expansion).
+static double form_us(int form, int fmt, int n, int K, int ng) {
+  const long g = (long)((n + FORM_ROWS[form] - 1) / FORM_ROWS[form]) * ((ng + FORM_GROUPS[form] - 1) / FORM_GROUPS[form]);
+  const double u = K / 128;
+  const double waves = (double)((g + 255) / 256);               // rounds at one workgroup per CU
+  const double pairs = (double)(g / 512 + (g % 512 > 256));     // at two, but for
+  const double tail = g % 512 != 0 && g % 512 <= 256;           // a last one of one per CU
+  switch (form) {
+    case F4_TILE: {   // 16 column blocks are one memory round trip
+      const double trip = fmt == FMT_Q1 ? 3.6 : fmt == FMT_Q2 ? 4.0 : 4.7;
+      return 1.1 + waves * trip * ((K + 2047) / 2048);
+    }
+    case F4_ROWS:   // unpacks its weights in every workgroup: by format
+      if (fmt == FMT_Q1) return 2.8 + (g <= 256 ? 0.64 * u : pairs * (0.18 + 0.77 * u) + tail * 0.435 * u);
+      if (fmt == FMT_Q2) return 2.5 + (g <= 256 ? 0.74 * u : pairs * (0.2 + 0.925 * u) + tail * 0.52 * u);
+      return 2.0 + (g <= 256 ? 1.24 * u : 0.26 * u + pairs * (0.4 + 1.33 * u) + tail * 0.5 * u);
+    case X_128x64_8: return 0.9 + waves * (4.3 + 0.54 * u);
+    case X_128x64_4: return 3.7 + tail * (1.4 + 0.63 * u) + pairs * (5.6 + 0.946 * u);
+    case X_128x128: return 3.7 + tail * (1.4 + 1.11 * u) + pairs * (5.6 + 1.777 * u);
+    default: return waves * (11.3 + 1.68 * u);
+  }
+}
+
+// Expanded weights: the whole matrix's where they fit F4X_SLAB, else that many rows
+// at a time.  An expansion reads its blocks and writes 2112 bytes per 32 x 128.
+constexpr size_t F4X_SLAB = (size_t)128 << 20;
 static int slab_rows(int n, int K) {   // rows per expansion: whole 256-row tiles
   const size_t per = (size_t)(K / 128) * 8 * WT_BYTES;
   return (int)std::min<size_t>((n + 255) / 256, std::max<size_t>(1, F4X_SLAB / per)) * 256;
 }
+static double expand_us(int n, int K) { return 2.0 + 0.16e-6 * n * K; }
+static int best_expanded(int fmt, int n, int K, int ng) {
+  int best = X_128x64_8;
+  for (int f = best + 1; f < N_FORMS; ++f)
+    if (form_us(f, fmt, n, K, ng) < form_us(best, fmt, n, K, ng)) best = f;
+  return best;
+}
+
+// The form without expanded weights, and the one that is chosen (for the first slab).
+static int direct_form(int fmt, int n, int K, int ng) {
+  // past 16 rounds the row form always wins
+  if ((long)((n + 31) / 32) * ng > 4096) return F4_ROWS;
+  return form_us(F4_TILE, fmt, n, K, ng) < form_us(F4_ROWS, fmt, n, K, ng) ? F4_TILE : F4_ROWS;
+}
+static int choose_form(int fmt, int n, int K, int seq) {
+  const int ng = (seq + 31) / 32, direct = direct_form(fmt, n, K, ng);
+  if (ng < 2) return direct;   // one group leaves half of every expanded tile empty
+  // (a grid dimension holds 2^32 lanes: the row form's tiles may be more)
+  const bool fits = (long)((n + 127) / 128) * ng < (1l << 24);
+  const double limit = fits ? form_us(direct, fmt, n, K, ng) : 1e30;
+  const int slab = slab_rows(n, K);
+  double us = 0.0;
+  for (int r0 = 0; r0 < n && us < limit; r0 += slab) {
+    const int nr = std::min(slab, n - r0);
+    us += expand_us(nr, K) + form_us(best_expanded(fmt, nr, K, ng), fmt, nr, K, ng);
+  }
+  return us < limit ? best_expanded(fmt, std::min(slab, n), K, ng) : direct;
+}
+
+// The chosen form and its rows per pass (fewer than n: expanded in slabs).
+int hh_gemm_f4_plan(int fmt, int n, int K, int seq, int* rows) {
+  const int form = choose_form(fmt, n, K, seq);
+  *rows = form >= X_128x64_8 ? std::min(slab_rows(n, K), n) : n;
+  return form;
+}
 
 size_t hh_gemm_f4_wbytes(int fmt, int n, int K, int seq) {
-  return expands(fmt, n, seq) ? (size_t)(slab_rows(n, K) / 32) * (K / 128) * WT_BYTES : 0;
+  return choose_form(fmt, n, K, seq) >= X_128x64_8 ? (size_t)(slab_rows(n, K) / 32) * (K / 128) * WT_BYTES : 0;
 }
 
 int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* tiles, int seq, uint8_t* wtiles,
@@ -676,8 +735,10 @@ int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* ti
   if (K <= 0 || K % 128 != 0 || n <= 0 || seq <= 0 || (fmt != FMT_Q2 && fmt != FMT_Q1 && fmt != FMT_PT)) return 1;
   const int ng = (seq + 31) / 32, ngp = act_groups(seq);
   const int vec = n % 4 == 0 && ((uintptr_t)out & 15) == 0;
-  if (!expands(fmt, n, seq) || !wtiles) {
-    const bool small = single_tiles(n, ng);
+  int form = choose_form(fmt, n, K, seq);
+  if (form >= X_128x64_8 && !wtiles) form = direct_form(fmt, n, K, ng);
+  if (form < X_128x64_8) {
+    const bool small = form == F4_TILE;
     const dim3 grid(small ? (unsigned)((n + 31) / 32) * ng : (unsigned)((n + 127) / 128) * ng);
 #define HH_F4(F)                                                                                                   \
   if (small) hipLaunchKernelGGL((k_gemm_f4s<F>), grid, dim3(512), 0, s, w, tiles, out, n, K, seq, ngp, vec);        \
@@ -700,28 +761,16 @@ int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* ti
     else if (fmt == FMT_Q1) HH_WT(FMT_Q1);
     else HH_WT(FMT_PT);
 #undef HH_WT
-    // The workgroup tile with the least time for this grid on 256 CUs, from the
-    // measured time of one 128-column step with a CU's workgroups resident, their start
-    // and stores spread over 32 steps (us):
-    //   256 x 128 (rows x tokens), 1 per CU : 2.5
-    //   128 x 128, 2 per CU : 2.6 (1.35 alone)
-    //   128 x 64, 2 per CU, 4 waves : 1.33 (0.9 alone); 8 waves, 1 per CU : 0.8
-    auto wgs = [&](int r, int t) { return (long)((nr + r - 1) / r) * ((ng + t - 1) / t); };
-    auto rounds = [](long g, double pair, double alone) {
-      const long full = g / 512, rest = g % 512;
-      return full * pair + (rest == 0 ? 0.0 : rest <= 256 ? alone : pair);
-    };
-    const double ta = ((wgs(256, 4) + 255) / 256) * 2.5, tb = rounds(wgs(128, 4), 2.6, 1.35);
-    const double tc = rounds(wgs(128, 2), 1.33, 0.9), td = ((wgs(128, 2) + 255) / 256) * 0.8;
-    const double best = std::min(std::min(ta, tb), std::min(tc, td));
 #define HH_F4X(RT, TT, WR, WT, NS)                                                                               \
   hipLaunchKernelGGL((k_gemm_f4x<RT, TT, WR, WT, NS>),                                                           \
                      dim3((nr + 32 * RT * WR - 1) / (32 * RT * WR), (ng + TT * WT - 1) / (TT * WT)),             \
                      dim3(64 * WR * WT), 0, s, wtiles, tiles, out, r0, n, K, seq, rg, ngp, vec)
-    if (best == td) HH_F4X(1, 1, 4, 2, 4);
-    else if (best == tc) HH_F4X(2, 1, 2, 2, 3);
-    else if (best == tb) HH_F4X(2, 2, 2, 2, 2);
-    else HH_F4X(4, 1, 2, 4, 3);
+    switch (best_expanded(fmt, nr, K, ng)) {
+      case X_128x64_8: HH_F4X(1, 1, 4, 2, 4); break;
+      case X_128x64_4: HH_F4X(2, 1, 2, 2, 3); break;
+      case X_128x128: HH_F4X(2, 2, 2, 2, 2); break;
+      default: HH_F4X(4, 1, 2, 4, 3);
+    }
 #undef HH_F4X
     if (hipGetLastError() != hipSuccess) return 1;
   }

@@ -842,15 +842,33 @@ int hh_gemv_q8(hh_ctx* c, int type, const void* w, int64_t n_rows, int64_t n_col
   return HH_OK;
 }
 
-int hh_gemm_q8(hh_ctx* c, int type, const void* w, int64_t n_rows, int64_t n_cols, const uint8_t* xq8,
-               int64_t seq_len, float* out) {
-  if (!c || !w || !xq8 || !out) return fail(HH_ERR_INVALID, "null argument");
-  int fmt = hh_fmt_of(type);
-  if (fmt < 0) return fail(HH_ERR_DTYPE, "unsupported weight dtype for the Q8_0 GEMM");
+static int gemm_args(int type, int64_t n_rows, int64_t n_cols, int64_t seq_len, int* fmt) {
+  *fmt = hh_fmt_of(type);
+  if (*fmt < 0) return fail(HH_ERR_DTYPE, "unsupported weight dtype for the Q8_0 GEMM");
   if (n_cols <= 0 || n_cols % 128 != 0) return fail(HH_ERR_DIM, "n_cols must be a positive multiple of 128");
+  if (n_cols > (1ll << 31) - 1) return fail(HH_ERR_DIM, "n_cols too large");   // the kernels count columns in 32 bits
   if (n_rows <= 0 || n_rows > (1ll << 30) || seq_len <= 0 || seq_len > (1ll << 24))
     return fail(HH_ERR_DIM, "bad n_rows or seq_len");
   if ((n_rows + 63) / 64 > 2147483647ll || (seq_len + 63) / 64 > 65535) return fail(HH_ERR_DIM, "grid too large");
+  return HH_OK;
+}
+
+int hh_gemm_q8_plan(int type, int64_t n_rows, int64_t n_cols, int64_t seq_len, int* form, int64_t* rows_per_pass) {
+  if (!form || !rows_per_pass) return fail(HH_ERR_INVALID, "null argument");
+  int fmt, rows = (int)n_rows;
+  const int rc = gemm_args(type, n_rows, n_cols, seq_len, &fmt);
+  if (rc != HH_OK) return rc;
+  *form = fmt == FMT_Q8 ? 6 : hh_gemm_f4_plan(fmt, (int)n_rows, (int)n_cols, (int)seq_len, &rows);
+  *rows_per_pass = rows;
+  return HH_OK;
+}
+
+int hh_gemm_q8(hh_ctx* c, int type, const void* w, int64_t n_rows, int64_t n_cols, const uint8_t* xq8,
+               int64_t seq_len, float* out) {
+  if (!c || !w || !xq8 || !out) return fail(HH_ERR_INVALID, "null argument");
+  int fmt;
+  const int rc = gemm_args(type, n_rows, n_cols, seq_len, &fmt);
+  if (rc != HH_OK) return rc;
   // scratch, grown on demand: activation tiles and, for many tokens, expanded
   // weights (1- and 2-bit formats), or int8 rows plus f32 block scales (Q8_0)
   const size_t nq = (size_t)seq_len * n_cols;

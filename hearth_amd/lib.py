@@ -141,6 +141,8 @@ _EXPORTS = {
     "hh_gemv_q8": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]),
     "hh_gemm_q8": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int64,
                              C.c_void_p]),
+    "hh_gemm_q8_plan": (C.c_int, [C.c_int, C.c_int64, C.c_int64, C.c_int64, C.POINTER(C.c_int),
+                                  C.POINTER(C.c_int64)]),
     "hh_rms_norm": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_float, C.c_int64, C.c_int64, C.c_void_p]),
     "hh_rope": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_int]),
     "hh_attention": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int,
@@ -247,6 +249,13 @@ def _ptrs(*xs):
                         stream.synchronize()
             out.append(x.data_ptr())
     return out
+
+
+def gemm_plan(ggml_type: int, n_rows: int, n_cols: int, seq_len: int) -> tuple:
+    """(form, rows per pass) of Ctx.gemm_q8's kernel for a product (hh_gemm_q8_plan); needs no device."""
+    form, rows = C.c_int(), C.c_int64()
+    _check(load_library().hh_gemm_q8_plan(ggml_type, n_rows, n_cols, seq_len, C.byref(form), C.byref(rows)))
+    return form.value, rows.value
 
 
 class Ctx:

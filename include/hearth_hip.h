@@ -106,6 +106,14 @@ int hh_gemv_q8(hh_ctx* ctx, int ggml_type, const void* w, int64_t n_rows, int64_
 int hh_gemm_q8(hh_ctx* ctx, int ggml_type, const void* w, int64_t n_rows, int64_t n_cols,
                const uint8_t* x_q8, int64_t seq_len, float* out);
 
+/* The kernel that hh_gemm_q8 and the prefill run for a product, asked without a
+ * device: *form 0 32 x 32 tiles (rows x tokens), 1 128 x 32; with the weights expanded
+ * first 2 128 x 64 by 8 waves, 3 128 x 64 by 4, 4 128 x 128, 5 256 x 128; 6 the int8
+ * kernel of Q8_0.  *rows_per_pass: rows expanded at a time, n_rows where one pass does
+ * them all.  Arguments are refused as hh_gemm_q8 refuses them. */
+int hh_gemm_q8_plan(int ggml_type, int64_t n_rows, int64_t n_cols, int64_t seq_len, int* form,
+                    int64_t* rows_per_pass);
+
 /* ops.rs:8-35 rms_norm over n_rows independent rows of width n. */
 int hh_rms_norm(hh_ctx* ctx, const float* x, const float* weight, float eps, int64_t n_rows,
                 int64_t n, float* out);

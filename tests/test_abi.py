@@ -50,6 +50,29 @@ def test_operator_pointers():
     assert tuple(_ptrs(x, None, 7, x)) == (x.data_ptr(), 0, 7, x.data_ptr())
 
 
+def test_gemm_plan():
+    """The GEMM's choice of a form needs no device: shallow products keep away from the
+    expanded forms, deep ones with many tokens take them, matrices past the expansion's
+    scratch in whole 256-row tiles; what the GEMM refuses is refused."""
+    from hearth_amd.lib import HHError, gemm_plan
+    for t in (41, 42, 143):
+        assert gemm_plan(t, 2048, 2048, 8) == (0, 2048)
+        assert gemm_plan(t, 24576, 1024, 64) == (1, 24576)
+        assert gemm_plan(t, 24576, 4096, 2048) == (4, 24576)
+        form, rows = gemm_plan(t, 34816, 17408, 2048)
+        assert form >= 2 and rows < 34816 and rows % 256 == 0
+        for seq in (1, 200, 1 << 20):   # the widest matrices and longest rows
+            assert gemm_plan(t, 1 << 30, 128, seq)[1] > 0 and gemm_plan(t, 1, (1 << 31) - 128, seq)[1] == 1
+    # int8 MFMA took 12.3 us: straight from the blocks 10.4, expanded 13.2
+    assert gemm_plan(42, 6144, 1024, 224) == (1, 6144)
+    assert gemm_plan(8, 4096, 4096, 512) == (6, 4096)
+    for args, status in (((2, 4, 128, 2), 2), ((42, 4, 100, 2), 3), ((42, 0, 128, 2), 3), ((42, 4, 128, 0), 3),
+                         ((42, 4, 1 << 32, 300), 3)):
+        with pytest.raises(HHError) as e:
+            gemm_plan(*args)
+        assert e.value.status == status
+
+
 def test_no_oracle_in_product():
     """The product package never imports or loads the oracle."""
     pkg = os.path.join(ROOT, "hearth_amd")

@@ -332,22 +332,17 @@ def test_gemm_bit_exact_vs_per_token_dot(ctx, oracle, t, n, k, seq):
 @pytest.mark.parametrize("t", [41, 42, 143])
 @pytest.mark.parametrize("n,k,seq", [
     (1, 128, 1), (33, 256, 32), (127, 2048, 33), (257, 2176, 255), (31, 4224, 65),   # one tile per workgroup
-    (24641, 256, 30), (12225, 384, 33), (8193, 128, 90),              # 128 rows per workgroup
-    (8200, 128, 224), (4097, 256, 257), (4226, 384, 300), (4096, 1024, 511),  # expanded, 128 x 64 by 8 waves; 1..8 steps
-    (4096, 128, 1024), (4095, 256, 1000),                             # 128 x 64 by 4 waves
-    (6144, 128, 2048), (4096, 384, 2048)])                            # 128 x 128 and 256 x 128
+    (24641, 256, 30), (12225, 384, 33), (8193, 128, 90), (12289, 1024, 33),
+    (8200, 128, 224), (4097, 256, 257), (4226, 384, 300), (4096, 1024, 511),
+    (4096, 128, 1024), (4095, 256, 1000), (6144, 128, 2048), (4096, 384, 2048)])
 def test_gemm_tiles_bit_exact(ctx, oracle, t, n, k, seq):
-    """Every tile shape of the 1- and 2-bit GEMM, at row, token and step counts around
-    its edges, on arbitrary codes, scales and activation bytes (-128 included): equal to
-    the scalar DotFn bit for bit on the tokens at tile edges."""
+    """The 1- and 2-bit GEMM at row, token and step counts around its tiles' edges, on
+    arbitrary codes, scales and activation bytes (-128 included): equal to the scalar
+    DotFn bit for bit on the tokens at tile edges."""
     print(f"gemm tiles t={t} n={n} k={k} seq={seq}", flush=True)
     rng = np.random.default_rng(n + k + seq + t)
     w = _random_weights(t, n, k, rng)
-    xq = rng.integers(0, 256, (seq * k // 32, 34), dtype=np.uint8)
-    sc = (rng.uniform(0, 2, len(xq)) * 10.0 ** rng.integers(-3, 2, len(xq))).astype(np.float16).view(np.uint16)
-    xq[:, 0], xq[:, 1] = sc & 0xFF, sc >> 8
-    xq = xq.reshape(seq, -1)
-    xq[seq - 1].reshape(-1, 34)[:, 2:] = 128
+    xq = _random_activations(seq, k, rng)
     out = torch.full((seq * n + 64,), 7.0, dtype=torch.float32, device="cuda")
     ctx.gemm_q8(t, dev(w), n, k, dev(xq.reshape(-1)), seq, out)
     got = host(out)
@@ -356,6 +351,49 @@ def test_gemm_tiles_bit_exact(ctx, oracle, t, n, k, seq):
     for s in sorted({v for e in range(0, seq + 32, 32) for v in (e - 1, e) if 0 <= v < seq and (seq < 600 or e % 512 == 0)}
                     | {seq - 1}):
         assert np.array_equal(got[s], oracle.gemv(t, w, n, k, xq[s])), s
+
+
+# (form, format, rows, columns, tokens, rows of one pass where they are fewer)
+FORMS = [
+    # 32 x 32 tiles: one round trip of 16 column blocks and an odd tail; three
+    (0, 42, 1023, 2176, 33, None), (0, 41, 257, 4224, 65, None), (0, 143, 127, 6016, 31, None),
+    # 128 x 32 straight from the blocks, 8 and 7 steps through its two buffers
+    (1, 41, 12289, 1024, 33, None), (1, 42, 12289, 1024, 33, None), (1, 143, 12289, 896, 33, None),
+    # expanded, 128 x 64 by 8 waves (ring of 4): 18 .. 20 and 23 steps
+    (2, 143, 4097, 2304, 33, None), (2, 143, 4097, 2432, 33, None), (2, 143, 4097, 2560, 33, None),
+    (2, 41, 2049, 2944, 511, None), (2, 42, 2049, 2176, 511, None),
+    # 128 x 64 by 4 waves (ring of 3): 5 .. 7 and 15 steps
+    (3, 143, 12289, 640, 257, None), (3, 143, 16385, 768, 161, None), (3, 143, 16385, 896, 161, None),
+    (3, 42, 16385, 1920, 161, None),
+    # 128 x 128 (ring of 2): 6, 7, 8 and 11 steps
+    (4, 143, 6145, 768, 333, None), (4, 143, 12289, 896, 161, None), (4, 42, 2049, 1024, 1500, None),
+    (4, 41, 2049, 1408, 1500, None),
+    # 256 x 128 (ring of 3): 21 .. 23 steps
+    (5, 42, 24577, 2688, 200, None), (5, 143, 24577, 2816, 200, None), (5, 42, 24577, 2944, 200, None)]
+
+
+@pytest.mark.parametrize("form,t,n,k,seq,slab", FORMS)
+def test_gemm_forms_bit_exact(ctx, oracle, form, t, n, k, seq, slab):
+    """Every form of the 1- and 2-bit GEMM over more steps than its buffers, at each
+    remainder of them: the form is the one meant, and the outputs at the edges of its
+    tiles equal the scalar DotFn bit for bit."""
+    from hearth_amd.lib import gemm_plan
+    assert gemm_plan(t, n, k, seq) == (form, slab or n)
+    print(f"gemm form={form} t={t} n={n} k={k} seq={seq}", flush=True)
+    rng = np.random.default_rng(n + k + seq + t)
+    w = _random_weights(t, n, k, rng)
+    xq = _random_activations(seq, k, rng)
+    out = torch.full((seq * n + 64,), 7.0, dtype=torch.float32, device="cuda")
+    ctx.gemm_q8(t, dev(w), n, k, dev(xq.reshape(-1)), seq, out)
+    got = host(out)
+    assert np.all(got[seq * n:] == 7.0)
+    got = got[:seq * n].reshape(seq, n)
+    edge = {v for e in range(0, n + 256, 256) for v in (e - 1, e, e + 31, e + 100)}
+    rows = np.array(sorted({v for v in edge if 0 <= v < n} | {n - 1}))
+    wr = np.ascontiguousarray(w.reshape(n, -1)[rows]).reshape(-1)
+    toks = {v for e in range(0, seq + 64, 64) for v in (e - 1, e, e + 32)} if seq < 600 else {0, 127, 128, 640, 1023, 1024}
+    for s in sorted({v for v in toks if 0 <= v < seq} | {seq - 1}):
+        assert np.array_equal(got[s, rows], oracle.gemv(t, wr, len(rows), k, xq[s])), s
 
 
 def test_gemm_errors(ctx):
@@ -381,6 +419,16 @@ def _random_weights(t, n_rows, n_cols, rng):
     blocks[:, off] = sc & 0xFF
     blocks[:, off + 1] = sc >> 8
     return w
+
+
+def _random_activations(seq, k, rng):
+    """Q8_0 rows of arbitrary bytes and scales of several decades; the last row is all -128."""
+    xq = rng.integers(0, 256, (seq * k // 32, 34), dtype=np.uint8)
+    sc = (rng.uniform(0, 2, len(xq)) * 10.0 ** rng.integers(-3, 2, len(xq))).astype(np.float16).view(np.uint16)
+    xq[:, 0], xq[:, 1] = sc & 0xFF, sc >> 8
+    xq = xq.reshape(seq, -1)
+    xq[seq - 1].reshape(-1, 34)[:, 2:] = 128
+    return xq
 
 
 from hypothesis import given, settings, strategies as hst   # noqa: E402
