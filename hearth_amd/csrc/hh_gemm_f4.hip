@@ -753,7 +753,7 @@ int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* ti
   }
   const int slab = slab_rows(n, K);
   for (int r0 = 0; r0 < n; r0 += slab) {
-    const int nr = std::min(slab, n - r0), rg = slab / 32;
+    const int nr = std::min(slab, n - r0), rg = (nr + 255) / 256 * 8;   // its own rows, in whole 256-row tiles
     const uint8_t* ws = w + (size_t)r0 * (K / 128) * (fmt == FMT_Q1 ? 18 : fmt == FMT_PT ? 28 : 34);
     const dim3 wgrid((K / 128 + 3) / 4, rg);
 #define HH_WT(F) hipLaunchKernelGGL((k_weight_tiles<F>), wgrid, dim3(256), 0, s, ws, nr, K, wtiles)

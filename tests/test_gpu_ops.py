@@ -353,7 +353,7 @@ def test_gemm_tiles_bit_exact(ctx, oracle, t, n, k, seq):
         assert np.array_equal(got[s], oracle.gemv(t, w, n, k, xq[s])), s
 
 
-# (form, format, rows, columns, tokens, rows of one pass where they are fewer)
+# (form, format, rows, columns, tokens), and the rows of one pass where they are fewer
 FORMS = [
     # 32 x 32 tiles: one round trip of 16 column blocks and an odd tail; three
     (0, 42, 1023, 2176, 33, None), (0, 41, 257, 4224, 65, None), (0, 143, 127, 6016, 31, None),
@@ -369,14 +369,17 @@ FORMS = [
     (4, 143, 6145, 768, 333, None), (4, 143, 12289, 896, 161, None), (4, 42, 2049, 1024, 1500, None),
     (4, 41, 2049, 1408, 1500, None),
     # 256 x 128 (ring of 3): 21 .. 23 steps
-    (5, 42, 24577, 2688, 200, None), (5, 143, 24577, 2816, 200, None), (5, 42, 24577, 2944, 200, None)]
+    (5, 42, 24577, 2688, 200, None), (5, 143, 24577, 2816, 200, None), (5, 42, 24577, 2944, 200, None),
+    # the weights expanded in slabs, the last of 153, 257 and (a third) 257 rows
+    (2, 143, 15001, 17408, 96, 14848), (5, 42, 15105, 17408, 400, 14848), (3, 143, 29953, 17408, 129, 14848)]
 
 
 @pytest.mark.parametrize("form,t,n,k,seq,slab", FORMS)
 def test_gemm_forms_bit_exact(ctx, oracle, form, t, n, k, seq, slab):
     """Every form of the 1- and 2-bit GEMM over more steps than its buffers, at each
-    remainder of them: the form is the one meant, and the outputs at the edges of its
-    tiles equal the scalar DotFn bit for bit."""
+    remainder of them, and over several slabs of expanded weights: the form is the one
+    meant, and the outputs at the edges of its tiles and slabs equal the scalar DotFn bit
+    for bit."""
     from hearth_amd.lib import gemm_plan
     assert gemm_plan(t, n, k, seq) == (form, slab or n)
     print(f"gemm form={form} t={t} n={n} k={k} seq={seq}", flush=True)
