@@ -94,8 +94,10 @@ struct hh_ctx {
   hipEvent_t ev[8] = {};
   void* attn_scratch = nullptr;     // standalone attention partials + counters
   size_t attn_scratch_bytes = 0;
-  void* gemm_scratch = nullptr;     // standalone GEMM: activations in split layout
+  uint8_t* gemm_scratch = nullptr;  // standalone GEMM: activation tiles and expanded weights, or split activations
   size_t gemm_scratch_bytes = 0;
+  size_t gemm_refused = ~(size_t)0; // the smallest size that was not to be had
+  size_t scratch_limit = ~(size_t)0; // hh_ctx_set_scratch_limit
 };
 
 namespace {
@@ -186,6 +188,7 @@ struct hh_model {
   // batched prefill scratch (grown on demand); HH_BATCHED_PREFILL=0 feeds prompts token by token
   uint8_t* pf_buf = nullptr;
   size_t pf_cap = 0;
+  size_t pf_refused = ~(size_t)0;   // the smallest size that was not to be had
   int batched_prefill = 1;
   // HH_GDN_CHUNKED=1: the batched prefill runs the GDN recurrence in chunked
   // form (fp32-rounding parity with the sequential rule instead of bit parity)
@@ -527,6 +530,49 @@ int ssm_a_all_negative(hh_model* m, bool* ok) {
   return HH_OK;
 }
 
+// A GEMM's scratch in falling sizes, for where memory is short: 0 all S tokens and the
+// expanded weights, 1 without these, then half the tokens at a time down to 128 (every
+// size gives the same bits).  False past the last.
+bool gemm_scratch_step(int i, int S, int* tokens, bool* expand) {
+  *expand = i == 0;
+  *tokens = S;
+  for (int k = 1; k < i; ++k) {
+    if (*tokens <= 128) return false;
+    *tokens = (*tokens / 2 + 127) / 128 * 128;
+  }
+  return true;
+}
+
+// Grow *buf to the first of the steps' sizes (bytes(i), falling) that is to be had;
+// returns that step, or -1.  A size that was refused once is not asked for again,
+// unless it is the last.
+template <class Bytes> int grow_scratch(const hh_ctx* c, uint8_t** buf, size_t* cap, size_t* refused, int n_steps,
+                                        Bytes bytes) {
+  for (int i = 0; i < n_steps; ++i) {
+    const size_t need = bytes(i);
+    if (need <= *cap) return i;
+    if (i + 1 < n_steps && need >= *refused) continue;
+    if (*buf) {
+      if (hipStreamSynchronize(c->stream) != hipSuccess || hipFree(*buf) != hipSuccess) return -1;
+      *buf = nullptr;
+      *cap = 0;
+    }
+    if (need <= c->scratch_limit && hipMalloc(buf, need) == hipSuccess) {
+      *cap = need;
+      return i;
+    }
+    *buf = nullptr;
+    (void)hipGetLastError();   // not the next launch's error
+    *refused = std::min(*refused, need);
+  }
+  return -1;
+}
+int gemm_scratch_steps(int S) {
+  int n = 1, t;
+  for (bool e; gemm_scratch_step(n, S, &t, &e);) ++n;
+  return n;
+}
+
 int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   const hh_model_config& c = m->cfg;
   hipStream_t s = m->ctx->stream;
@@ -564,25 +610,25 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   // attention's partials are never live together, so they share one region
   const size_t po = align256((size_t)TA * c.n_kv_heads * n_chunks * G * hd * 4);
   const size_t pml = (size_t)TA * c.n_kv_heads * n_chunks * G * 2 * 4;
-  const size_t act = align256(hh_act_tiles_bytes(kmax, S));
-  size_t off = 0;
+  const int steps = gemm_scratch_steps(S);
+  int ST = S;   // tokens per GEMM
+  bool expand = true;
+  size_t act = 0, off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align256(off + bytes); return o; };
   const size_t oH = take((size_t)S * d * 4), oXq = take((size_t)S * kmax), oXd = take((size_t)S * (kmax / 32) * 4),
                oQKV = take((size_t)S * n_in_max * 4), oQB = take((size_t)S * nq * 4),
                oT = take((size_t)S * d * 4), oGU = take((size_t)S * 2 * F * 4),
-               oPart = take(std::max(po + pml, act + wt_max)),
                oGQK = take(hyb ? (size_t)S * 2 * kdim * 4 : 0), oGV = take(hyb ? (size_t)S * vdim * 4 : 0),
                oGAB = take(hyb ? (size_t)S * 2 * c.ssm_n_v_heads * 4 : 0),
                oGDEC = take(hyb ? (size_t)S * c.ssm_n_v_heads * 4 : 0), oGO = take(hyb ? (size_t)S * vdim * 4 : 0),
                oRot = take(c.had_block > 0 ? (size_t)S * std::max(std::max(vdim, nq), F) * 4 : 0),
-               oChunk = take(hyb && chunked ? hh_gdn_chunk_scratch_bytes(c.ssm_n_v_heads, S) : 0);
-  if (off > m->pf_cap) {
-    if (m->pf_buf) HIP_TRY(hipFree(m->pf_buf));
-    m->pf_buf = nullptr;
-    m->pf_cap = 0;
-    if (hipMalloc(&m->pf_buf, off) != hipSuccess) return fail(HH_ERR_OOM, "prefill scratch allocation failed");
-    m->pf_cap = off;
-  }
+               oChunk = take(hyb && chunked ? hh_gdn_chunk_scratch_bytes(c.ssm_n_v_heads, S) : 0), oPart = off;
+  const int step = grow_scratch(m->ctx, &m->pf_buf, &m->pf_cap, &m->pf_refused, steps, [&](int i) {
+    gemm_scratch_step(i, S, &ST, &expand);
+    act = align256(hh_act_tiles_bytes(kmax, ST));
+    return oPart + std::max(po + pml, act + (expand ? wt_max : 0));
+  });
+  if (step < 0) return fail(HH_ERR_OOM, "prefill scratch allocation failed");
   uint8_t* B = m->pf_buf;
   float* H = (float*)(B + oH);
   int8_t* Xq = (int8_t*)(B + oXq);
@@ -604,8 +650,15 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
     return hh_norm_q8_rows_launch(H, w, c.eps, d, S, Xq, Xd, s);
   };
   auto gemm = [&](const uint8_t* w, int n, int K, float* out) -> int {
-    const int rc = hh_act_tiles_launch(m->wfmt, nullptr, Xq, Xd, K, S, Act, s);
-    return rc ? rc : hh_gemm_f4_launch(m->wfmt, w, n, K, Act, S, wt_max ? Act + act : nullptr, out, s);
+    for (int t0 = 0; t0 < S; t0 += ST) {
+      const int nt = std::min(ST, S - t0);
+      const int8_t* xq = Xq + (size_t)t0 * K;
+      const float* xd = Xd + (size_t)t0 * (K / 32);
+      if (const int rc = hh_act_tiles_launch(m->wfmt, nullptr, xq, xd, K, nt, Act, s)) return rc;
+      uint8_t* wt = expand && wt_max ? Act + act : nullptr;
+      if (const int rc = hh_gemm_f4_launch(m->wfmt, w, n, K, Act, nt, wt, out + (size_t)t0 * n, s)) return rc;
+    }
+    return 0;
   };
   KTRY(hh_embed_rows_launch(c.head_type, m->token_embd->d, d, toks, S, H, latent ? signs_of(m, d) : nullptr,
                             latent ? c.had_block : 0, s));
@@ -731,6 +784,12 @@ int hh_ctx_create(int device_ordinal, hh_ctx** out) {
     return fail(rc, msg);
   }
   *out = c;
+  return HH_OK;
+}
+
+int hh_ctx_set_scratch_limit(hh_ctx* c, uint64_t bytes) {
+  if (!c) return fail(HH_ERR_INVALID, "null argument");
+  c->scratch_limit = bytes ? (size_t)bytes : ~(size_t)0;
   return HH_OK;
 }
 
@@ -869,36 +928,38 @@ int hh_gemm_q8(hh_ctx* c, int type, const void* w, int64_t n_rows, int64_t n_col
   int fmt;
   const int rc = gemm_args(type, n_rows, n_cols, seq_len, &fmt);
   if (rc != HH_OK) return rc;
-  // scratch, grown on demand: activation tiles and, for many tokens, expanded
-  // weights (1- and 2-bit formats), or int8 rows plus f32 block scales (Q8_0)
-  const size_t nq = (size_t)seq_len * n_cols;
-  const size_t act = align256(fmt == FMT_Q8 ? nq : hh_act_tiles_bytes((int)n_cols, (int)seq_len));
-  const size_t extra = fmt == FMT_Q8 ? nq / 32 * 4 : hh_gemm_f4_wbytes(fmt, (int)n_rows, (int)n_cols, (int)seq_len);
-  if (c->gemm_scratch_bytes < act + extra) {
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (c->gemm_scratch) HIP_TRY(hipFree(c->gemm_scratch));
-    c->gemm_scratch = nullptr;
-    c->gemm_scratch_bytes = 0;
-    size_t got = act + extra;
-    if (hipMalloc(&c->gemm_scratch, got) != hipSuccess) {
-      c->gemm_scratch = nullptr;
-      (void)hipGetLastError();
-      got = fmt == FMT_Q8 ? got : act;   // the product runs without the expanded weights too
-      HIP_TRY(hipMalloc(&c->gemm_scratch, got));
-    }
-    c->gemm_scratch_bytes = got;
-  }
-  uint8_t* buf = (uint8_t*)c->gemm_scratch;
-  if (fmt != FMT_Q8) {
-    KTRY(hh_act_tiles_launch(fmt, xq8, nullptr, nullptr, (int)n_cols, (int)seq_len, buf, c->stream));
-    KTRY(hh_gemm_f4_launch(fmt, (const uint8_t*)w, (int)n_rows, (int)n_cols, buf, (int)seq_len,
-                           extra && c->gemm_scratch_bytes >= act + extra ? buf + act : nullptr, out, c->stream));
+  // scratch, grown on demand: int8 rows plus f32 block scales (Q8_0), or activation
+  // tiles and, for many tokens, expanded weights (1- and 2-bit formats)
+  const int K = (int)n_cols, n = (int)n_rows, S = (int)seq_len;
+  if (fmt == FMT_Q8) {
+    const size_t nq = (size_t)S * K, act = align256(nq);
+    if (grow_scratch(c, &c->gemm_scratch, &c->gemm_scratch_bytes, &c->gemm_refused, 1,
+                     [&](int) { return act + nq / 32 * 4; }) < 0)
+      return fail(HH_ERR_HIP, "GEMM scratch allocation failed");
+    int8_t* xq = (int8_t*)c->gemm_scratch;
+    float* xd = (float*)(c->gemm_scratch + act);
+    KTRY(hh_q8_split_launch(xq8, (int64_t)(nq / 32), xq, xd, c->stream));
+    KTRY(hh_gemm_launch((const uint8_t*)w, n, K, xq, xd, S, out, c->stream));
     return HH_OK;
   }
-  int8_t* xq = (int8_t*)buf;
-  float* xd = (float*)(buf + act);
-  KTRY(hh_q8_split_launch(xq8, (int64_t)(nq / 32), xq, xd, c->stream));
-  KTRY(hh_gemm_launch((const uint8_t*)w, (int)n_rows, (int)n_cols, xq, xd, (int)seq_len, out, c->stream));
+  const size_t wt = hh_gemm_f4_wbytes(fmt, n, K, S);
+  int ST = S;   // tokens per pass
+  bool expand = true;
+  size_t act = 0;
+  const int step = grow_scratch(c, &c->gemm_scratch, &c->gemm_scratch_bytes, &c->gemm_refused, gemm_scratch_steps(S),
+                                [&](int i) {
+                                  gemm_scratch_step(i, S, &ST, &expand);
+                                  act = align256(hh_act_tiles_bytes(K, ST));
+                                  return act + (expand ? wt : 0);
+                                });
+  if (step < 0) return fail(HH_ERR_HIP, "GEMM scratch allocation failed");
+  uint8_t* buf = c->gemm_scratch;
+  for (int t0 = 0; t0 < S; t0 += ST) {
+    const int nt = std::min(ST, S - t0);
+    KTRY(hh_act_tiles_launch(fmt, xq8 + (size_t)t0 * (K / 32) * 34, nullptr, nullptr, K, nt, buf, c->stream));
+    KTRY(hh_gemm_f4_launch(fmt, (const uint8_t*)w, n, K, buf, nt, expand && wt ? buf + act : nullptr,
+                           out + (size_t)t0 * n, c->stream));
+  }
   return HH_OK;
 }
 

@@ -128,6 +128,7 @@ _EXPORTS = {
     "hh_version": (C.c_char_p, []),
     "hh_ctx_create": (C.c_int, [C.c_int, C.POINTER(C.c_void_p)]),
     "hh_ctx_destroy": (C.c_int, [C.c_void_p]),
+    "hh_ctx_set_scratch_limit": (C.c_int, [C.c_void_p, C.c_uint64]),
     "hh_ctx_synchronize": (C.c_int, [C.c_void_p]),
     "hh_malloc": (C.c_int, [C.c_void_p, C.c_size_t, C.POINTER(C.c_void_p)]),
     "hh_free": (C.c_int, [C.c_void_p, C.c_void_p]),

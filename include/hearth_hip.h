@@ -65,6 +65,11 @@ const char* hh_version(void);
 /* ---- context: replaces GpuCompute::new() -> Option<Self> (hearth-compute lib.rs:126) ---- */
 int hh_ctx_create(int device_ordinal, hh_ctx** out);
 int hh_ctx_destroy(hh_ctx* ctx);
+/* The most bytes that one growth of the context's GEMM scratch, or of a prefill's, may
+ * ask for from now on (0: no limit, the default).  Both make do with less, slower and
+ * with the same results: without expanded weights, then with fewer tokens at a time;
+ * past that a call fails as if the memory were not there. */
+int hh_ctx_set_scratch_limit(hh_ctx* ctx, uint64_t bytes);
 int hh_ctx_synchronize(hh_ctx* ctx);
 /* Device memory helpers (GpuCompute::upload_bytes / readback_f32, lib.rs:230-243). */
 int hh_malloc(hh_ctx* ctx, size_t nbytes, void** dptr);

@@ -399,6 +399,76 @@ def test_gemm_forms_bit_exact(ctx, oracle, form, t, n, k, seq, slab):
         assert np.array_equal(got[s, rows], oracle.gemv(t, wr, len(rows), k, xq[s])), s
 
 
+def _limited_ctx(limit):
+    from hearth_amd import Ctx
+    from hearth_amd.lib import _check
+    c = Ctx(0)
+    _check(c.lib.hh_ctx_set_scratch_limit(c.h, int(limit)))
+    return c
+
+
+def test_gemm_short_of_memory():
+    """A product that wants expanded weights runs without them, and then in passes of
+    fewer tokens, where its scratch is not to be had: the same bits; less than 128
+    tokens' tiles is an error, and the context works on afterwards."""
+    from hearth_amd import HHError
+    from hearth_amd.lib import gemm_plan
+    n, k, seq = 2049, 2176, 511
+    tiles = [k // 128 * (s // 32) * 6656 for s in (512, 256, 128)]
+    assert gemm_plan(42, n, k, seq) == (2, n)
+    rng = np.random.default_rng(5)
+    w, xq = dev(_random_weights(42, n, k, rng)), dev(_random_activations(seq, k, rng).reshape(-1))
+    want = None
+    for limit in (0, tiles[0] + 256, tiles[1], tiles[2]):
+        c = _limited_ctx(limit)
+        print(f"gemm scratch limit {limit}", flush=True)
+        for s in (seq, seq, 40, seq):
+            out = torch.full((s * n + 64,), 7.0, dtype=torch.float32, device="cuda")
+            c.gemm_q8(42, w, n, k, xq, s, out)
+            got = host(out)
+            want = got if want is None else want
+            assert np.array_equal(got[:s * n], want[:s * n]) and np.all(got[s * n:] == 7.0)
+        c.close()
+    c = _limited_ctx(tiles[2] - 1)
+    with pytest.raises(HHError):
+        c.gemm_q8(42, w, n, k, xq, seq, out)
+    c.lib.hh_ctx_set_scratch_limit(c.h, 0)
+    out.fill_(7.0)
+    c.gemm_q8(42, w, n, k, xq, seq, out)
+    assert np.array_equal(host(out)[:seq * n], want[:seq * n])
+    c.close()
+
+
+def test_prefill_short_of_memory():
+    """The same for a model's prefill, whose GEMMs share one scratch."""
+    from hearth_amd import GGML_Q2_0, HHError, Model, ModelConfig
+    cfg = ModelConfig(d_model=2048, n_layers=2, n_heads=4, n_kv_heads=2, head_dim=128, d_ffn=12288, vocab=2048,
+                      max_seq=512, wtype=GGML_Q2_0)
+    prompt = np.random.default_rng(6).integers(0, cfg.vocab, 301).astype(np.uint32)
+
+    def run(limit):
+        c = _limited_ctx(limit)
+        m = Model(c, cfg)
+        m.synthesize(3)
+        print(f"prefill scratch limit {limit}", flush=True)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        try:
+            toks, logits = m.generate(prompt, 2, want_logits=True)
+            return list(toks), logits.copy(), free - torch.cuda.mem_get_info()[0]
+        finally:
+            m.close()
+            c.close()
+    toks, logits, used = run(0)
+    # 26 MB of it are expanded weights (24576 x 2048), 7.7 MB the tiles of 300 tokens
+    for limit in (used - (5 << 20), used - (28 << 20)):
+        t, lg, less = run(limit)
+        assert t == toks and np.array_equal(lg, logits)
+        assert less < used
+    with pytest.raises(HHError):
+        run(1 << 20)
+
+
 def test_gemm_errors(ctx):
     from hearth_amd import HHError
     w = torch.zeros(4096, dtype=torch.uint8, device="cuda")
