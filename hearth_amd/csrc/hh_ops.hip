@@ -1153,7 +1153,10 @@ __global__ __launch_bounds__(64 * NWV, 2) void k_attn_prefill_split(const float*
   static_assert(QS * NP == NWV && (QS == 1 || QS == 2) && (EW == 1 || EW == 2 || EW == 4), "wave split");
   constexpr int QL = HB * 16 * HD / 4 / (64 * NWV);   // 16-byte copies of q per lane and batch
   __shared__ float sm_m[HB][NP][16];
-  __shared__ __align__(16) float sm_e[HB][64][ES];   // [token * 4 + g]; row stride 16 (2 k + 1) bytes: no conflicts
+  // [token * 4 + g]: a lane group's 16-byte accesses are 4 rows apart and meet four ways on
+  // the 64 banks (35.7 M conflict cycles over 7.16 M LDS instructions for 2048 tokens of an
+  // 8B layer, about 11% of its CU cycles)
+  __shared__ __align__(16) float sm_e[HB][64][ES];
   // q, 1 KB copies: two tokens' units interleaved (hd 128) or one token (hd 256), padded
   // so that 16 tokens' reads of one slice fall on 64 banks
   constexpr int QP = HD == 128 ? 264 : 260;

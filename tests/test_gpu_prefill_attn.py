@@ -10,7 +10,7 @@ restatement of causal softmax attention:
     float64 (its sums are regrouped, so this is its parity bar).
 
 Geometries cover head_dim 128 and 256, query groups 1, 3, 4, 6 and 8 (so the
-MFMA kernel's 4 tiles and 1 tile per workgroup), partial 16-token tiles, a
+MFMA kernel's workgroups of 4 tiles and of 1 tile; 2 tiles are tested below), partial 16-token tiles, a
 prompt that starts past position 0 and one long enough for many chunks.  A
 model-level check runs a 9B-shaped slice and an 8B-shaped slice through the
 batched prefill both ways."""
