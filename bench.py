@@ -1,6 +1,6 @@
 """Benchmark: batch-1 greedy decode of the 8B-shaped Q2_0 model at 2k context.
 
-Workload (the north-star config): d_model 4096, 36
+Workload (the 8B Q2_0 decoder at 2k context): d_model 4096, 36
 layers, 32 q / 8 kv heads x 128, SwiGLU 12288, vocab 151936; Q2_0 layer weights
 and Q8_0 embedding/head synthesized on the device from a seed; f32 KV cache
 pre-filled at positions 0..2047 with seeded N(0,1) values rounded to fp16; then
@@ -238,7 +238,7 @@ def single_leg(ctx, name: str) -> dict:
 
 
 def config_legs(ctx) -> dict:
-    """BASELINE configs[0], [1], [3], [4] on the device (seeded synthetic weights).
+    """The 1.7B, GEMV, 9B and 27B workloads on the device (seeded synthetic weights).
     The prompt phase includes the last prompt token's decode step."""
     from hearth_amd import CONFIGS, microbench
     out = {}
@@ -345,12 +345,12 @@ def main():
                     help="batched-prefill leg after the decode measurement (0 = skip)")
     ap.add_argument("--no-hybrid", action="store_true", help="skip the 9B hybrid prefill + decode leg")
     ap.add_argument("--no-configs", action="store_true",
-                    help="skip the BASELINE configs[0,1,3,4] legs (1.7B Q1_0, GEMV microbench, 9B and 27B hybrids)")
+                    help="skip the other legs (1.7B Q1_0, GEMV microbench, 9B and 27B hybrids)")
     ap.add_argument("--hybrid-only", action="store_true",
                     help="run only the 9B hybrid leg and print its JSON (profiling)")
     ap.add_argument("--leg", choices=("1.7b", "9b", "27b", "27b-decode"), default=None,
-                    help="run only one configs leg (1.7B Q1_0 = configs[0], 9B hybrid = configs[3], "
-                         "27B hybrid = configs[4]; 27b-decode: the 27B at 8192 context with a 64-token "
+                    help="run only one of the other legs (1.7B Q1_0, 9B hybrid, "
+                         "27B hybrid; 27b-decode: the 27B at 8192 context with a 64-token "
                          "prompt and 16 decode steps, for counter runs) and print its JSON (profiling)")
     args = ap.parse_args()
     if args.gpus != 1:

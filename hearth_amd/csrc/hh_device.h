@@ -76,7 +76,7 @@ HH_DEV uint32_t f2h(float xf) {
 // two-step power-of-two scale (inputs below -87.33, whose results would be
 // subnormal, give 0); log via m = 2^-e x in [sqrt(1/2), sqrt(2)),
 // s = (m-1)/(m+1), log m = 2 atanh(s) (odd series to s^13).  Every step is an
-// IEEE single operation with explicit fmaf, so the CPU checker evaluates the
+// IEEE single operation with explicit fmaf, so the CPU reference evaluates the
 // identical function bit for bit.  Accuracy ~1-2 ulp (tested against libm).
 HH_DEV float hx_exp(float x_in) {
   // branch-free: the range cases are selected at the end, the polynomial runs
@@ -367,7 +367,7 @@ HH_DEV int grouped_pos(int e, int hd, int nk, int rep) {
   return ((h % nk) * rep + h / nk) * hd + (e - h * hd);
 }
 
-// ---- counter-based seeded generator (shared definition with the CPU checker) ----
+// ---- counter-based seeded generator (shared definition with the CPU reference) ----
 HH_DEV uint64_t mix64(uint64_t x) {
   x ^= x >> 30;
   x *= 0xbf58476d1ce4e5b9ull;

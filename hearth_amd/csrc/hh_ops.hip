@@ -1952,7 +1952,7 @@ __global__ void k_count_tokens(const uint32_t* past, int64_t n, int* counts) {
 
 // Measurement: stream n16 16-byte words, 8 loads in flight per lane, and keep
 // nothing (the store needs a sum no launch produces: `never` is -1).  Its rate
-// is the read-only HBM ceiling the decode step's streams are judged against.
+// is the read-only HBM ceiling the decode step's streams are held against.
 __global__ __launch_bounds__(1024) void k_read_probe(const uint4* __restrict__ p, int64_t n16, int* sink, int never) {
   uint32_t acc = 0;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -1973,7 +1973,7 @@ __global__ void k_fill_i32(int* p, int64_t n, int v) {
 }
 
 // ---------------------------------------------------------------------------
-// Seeded synthetic tensors (same definition as the CPU checker in tests).
+// Seeded synthetic tensors (same definition as the CPU reference in tests).
 // ---------------------------------------------------------------------------
 __global__ void k_synth_f32(uint64_t key, int64_t n, float c, float mean, float* out) {
 #pragma clang fp contract(off)

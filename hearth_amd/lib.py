@@ -71,7 +71,7 @@ class ModelConfigC(C.Structure):
 
 @dataclasses.dataclass
 class ModelConfig:
-    """hh_model_config / ho_config (the BASELINE.json model geometries)."""
+    """hh_model_config / ho_config (a model geometry)."""
     arch: int = 0
     d_model: int = 2048
     n_layers: int = 28
@@ -104,9 +104,8 @@ class ModelConfig:
         return dataclasses.replace(self, **kw)
 
 
-# BASELINE.json configs.  Head/embedding Q8_0 everywhere.  The 9B/27B hybrids use
-# partial RoPE over 64 of 256 dims; the 27B attention/GDN head counts are not in
-# BASELINE and are stated here (24 q / 4 kv x 256; GDN 16 k / 32 v x 128).
+# The measured models.  Head/embedding Q8_0 everywhere.  The 9B/27B hybrids use
+# partial RoPE over 64 of 256 dims; the 27B has 24 q / 4 kv heads x 256.
 CONFIGS = {
     "1.7b-q1": ModelConfig(),
     "8b-q2": ModelConfig(d_model=4096, n_layers=36, n_heads=32, n_kv_heads=8, head_dim=128,

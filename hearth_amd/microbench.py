@@ -1,4 +1,4 @@
-"""GEMV microbenchmark: Q1_0 and Q2_0 GEMVs (and
+"""GEMV microbenchmark (6144 x 2048, 2048 x 6144, 151936 x 2048): Q1_0 and Q2_0 GEMVs (and
 PTQ1_0, the 28-byte ternary format) at the 1.7B shapes N x K = 6144x2048,
 2048x6144, 151936x2048, plus the 8B FFN shapes, on Q8_0 activations from
 N(0,1), 1000 repetitions.  Each repetition reads a different weight copy from a

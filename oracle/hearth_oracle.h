@@ -1,7 +1,7 @@
 /*
  * hearth_oracle.h — CPU restatement of Hearth's batch-1 decode path.
  *
- * TEST INFRASTRUCTURE ONLY.  This library is the parity checker for the HIP
+ * TEST INFRASTRUCTURE ONLY.  This library is the parity reference for the HIP
  * library in hearth_amd/ and the "port" CPU baseline timed by bench.py.  It is
  * never linked into, loaded by, or called from the product path.  Only tests/,
  * __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it.

@@ -1,7 +1,6 @@
 // test_host.cpp — tests of the C++ host side (hearth_amd/host/hearth_host.hpp),
 // written the way the reference's inline Rust tests read, through the C ABI and
-// checked against the CPU oracle (oracle/hearth_oracle.h, linked as the
-// checker only).
+// checked against the CPU oracle (oracle/hearth_oracle.h).
 //
 //   test_host --cpu    tests that need no device (the CPU suite runs these)
 //   test_host          every test (on a GPU box)

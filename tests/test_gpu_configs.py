@@ -1,7 +1,6 @@
-"""GPU parity at the BASELINE.json model geometries that the other model tests
-only slice: configs[0] (the full 1.7B Q1_0 dense model), configs[1] (the full
-8B Q2_0 model against the reference order) and configs[4] (the 27B PQ2_0
-hybrid geometry, a few layers, batched prefill at 8192 context).
+"""GPU parity at the measured model geometries that the other model tests
+only slice: the full 1.7B Q1_0 dense model, the full 8B Q2_0 model against
+the reference order and the 27B PQ2_0 hybrid (its geometry, a few layers, batched prefill at 8192 context).
 
 Bars: tokens and logits bit-identical to the device-order oracle (the HIP
 kernels' fp32 grouping), and, against the reference-order oracle, every greedy
@@ -31,7 +30,7 @@ def m17(ctx):
 
 
 def test_config0_1p7b_q1_device_order(ctx, oracle, m17):
-    """d 2048, 28 layers, 16/8 x 128, ffn 6144, vocab 151936, Q1_0
+    """1.7B: d 2048, 28 layers, 16/8 x 128, ffn 6144, vocab 151936, Q1_0
     layers, Q8_0 embedding/head; 16-token seeded prompt, 50 greedy tokens with
     the sampler's default repetition penalty 1.1 (core/sampler.rs:18)."""
     cfg = CONFIGS["1.7b-q1"]
@@ -47,7 +46,7 @@ def test_config0_1p7b_q1_device_order(ctx, oracle, m17):
 
 
 def test_config0_1p7b_q1_reference_order(ctx, oracle, m17):
-    """configs[0] against the reference-order oracle: 50 greedy steps (penalty
+    """The 1.7B against the reference-order oracle: 50 greedy steps (penalty
     1.1), teacher-forced on the reference's sequence."""
     from tokcheck import reference_run, check_candidate, ambiguous_steps
     cfg = CONFIGS["1.7b-q1"]
@@ -64,7 +63,7 @@ def test_config0_1p7b_q1_reference_order(ctx, oracle, m17):
 
 
 def test_config4_27b_pq2_prefill_decode(ctx, oracle):
-    """configs[4] geometry (d 5120, ffn 17408, 24/4 x 256 attention with the
+    """27B geometry (d 5120, ffn 17408, 24/4 x 256 attention with the
     gate, GDN 16 k / 32 v x 128, vocab 248320, PQ2_0) with 4 layers (3 GDN + 1
     full attention) at max_seq 8192: a 320-token batched prefill on the MFMA
     GEMM, then 16 greedy decode steps.  Tokens and final logits equal the
@@ -86,7 +85,7 @@ def test_config4_27b_pq2_prefill_decode(ctx, oracle):
 
 
 def test_config1_8b_reference_order(ctx, oracle):
-    """configs[1], the benchmarked workload itself: the full 36-layer 8B Q2_0
+    """The 8B, the benchmarked workload itself: the full 36-layer 8B Q2_0
     model, KV pre-filled to 2048 positions, 32 greedy steps with the 1.1
     penalty, teacher-forced on the reference-order oracle's own sequence (the
     first-32-tokens bar, at full depth).  Random synthetic weights give nearly
@@ -128,7 +127,7 @@ def test_config1_8b_reference_order(ctx, oracle):
 
 
 def test_config3_9b_full_depth_prefill(ctx, oracle):
-    """configs[3] at full depth: the 9B-shaped qwen35 hybrid (32 layers: 24
+    """The 9B at full depth: the 9B-shaped qwen35 hybrid (32 layers: 24
     Gated-DeltaNet + 8 gated full attention, 16/4 x 256, GDN 16 k / 32 v x 128,
     vocab 248320, Q2_0), a 96-token seeded prompt through the batched prefill
     (MFMA GEMMs, GDN rows kernels, gated prefill attention), then 8 greedy
@@ -155,7 +154,7 @@ def test_config3_9b_full_depth_prefill(ctx, oracle):
 
 
 def test_config4_27b_16_layers_512_prefill(ctx, oracle):
-    """configs[4] geometry (d 5120, ffn 17408, 24/4 x 256 gated attention, GDN
+    """27B geometry (d 5120, ffn 17408, 24/4 x 256 gated attention, GDN
     16 k / 32 v x 128, vocab 248320, PQ2_0) with 16 of its 64 layers (12 GDN +
     4 full attention) at max_seq 8192: a 512-token batched prefill, then 8
     greedy decode steps; tokens and last logits equal the device-order oracle

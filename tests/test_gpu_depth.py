@@ -1,5 +1,5 @@
 """Logit agreement with the reference by depth on the benchmarked 8B geometry
-(configs[2]: d 4096, 32/8 x 128, ffn 12288, vocab 151936, Q2_0), the device
+(d 4096, 32/8 x 128, ffn 12288, vocab 151936, Q2_0), the device
 measured at 1, 2, 4, 9, 18 and 36 layers.  Synthesis is keyed by tensor name,
 so the models share their first layers; each runs 4 teacher-forced steps from
 position 2048 over the same synthetic KV cache.
@@ -11,7 +11,7 @@ Per step and depth:
     oracle (the reference's own arithmetic, ops.rs / q2_0.rs:537-574, on the
     device's quantized inputs) reproduces the device's logits within 1e-5;
   * while no Q8_0 byte has flipped against the reference's scalar arm, the
-    device meets the north-star bar (1e-3 relative); every larger deviation
+    device meets the bar (1e-3 relative); every larger deviation
     has a flip behind it.
 The reference's AVX2 arm (q2_0.rs:308-392) is measured beside it on the same
 inputs.  The table is printed (pytest -s)."""

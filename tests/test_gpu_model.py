@@ -1,6 +1,6 @@
 """GPU parity of whole decode steps and the token loop against the CPU oracle.
 
-Bars (north star): synthesized weight bytes bit-exact; logits within 1e-3
+Bars: synthesized weight bytes bit-exact; logits within 1e-3
 relative (max |diff| / max |ref|); greedy tokens identical for the first 32.
 
 The oracle runs in its device association order (the HIP kernels' reduction

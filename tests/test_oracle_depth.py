@@ -8,7 +8,7 @@ are ~1e-7 relative; they matter only where they move an activation across a
 Q8_0 rounding boundary (a byte, or the f16 block scale), and one such flip is
 a quantum of amax/127 that the layers after it carry forward.
 
-These checks run on the 8B geometry (configs[2]: d 4096, 32/8 x 128, ffn
+These checks run on the 8B geometry (d 4096, 32/8 x 128, ffn
 12288, vocab 151936) truncated to 1 and 2 layers, 8 teacher-forced steps from
 position 2048 over the synthetic KV cache, with the oracle in the device's
 order (bit-identical to the HIP library, tests/test_gpu_depth.py) and in the
@@ -17,7 +17,7 @@ reference's order:
     model (its own arithmetic, the device's quantized inputs) reproduces the
     device's logits within 1e-5 at every step: all of the difference is flips;
   * while no byte has flipped (this step or an earlier one, through the KV
-    cache), the device meets the north-star 1e-3 logit bar against the
+    cache), the device meets the 1e-3 logit bar against the
     reference's scalar arm; every step beyond 1e-3 has a flip behind it;
   * the reference's own AVX2 arm (q2_0.rs:308-392) behaves the same way:
     replaying its bytes into the scalar arm reproduces it within 1e-5.
@@ -85,7 +85,7 @@ def test_depth_deviation_is_q8_flips(oracle, L):
         seen += r["flips"]
         assert r["replay"] <= 1e-5, r              # the device's arithmetic, given its bytes
         if seen == 0:
-            assert r["dev"] <= 1e-3, r             # north-star bar while no byte has flipped
+            assert r["dev"] <= 1e-3, r             # the bar while no byte has flipped
         if r["dev"] > 1e-3:
             assert seen > 0, r                     # a deviation beyond the bar has a flip behind it
         if "avx" in r:
