@@ -227,11 +227,12 @@ def _ptrs(*xs):
     async fill or copy on torch's current stream of their device) is waited for
     first: once per device and call, and only where a query says that the stream is
     not idle (three synchronizations took 8 of the 11.7 us of a small gemv_q8)."""
-    for x in xs:
-        if type(x) is not int:
-            break
-    else:
-        return xs
+    if type(xs[0]) is int:   # raw addresses: nothing to wait for (tensors pay one test)
+        for x in xs:
+            if type(x) is not int:
+                break
+        else:
+            return xs
     out, waited = [], ()
     for x in xs:
         if isinstance(x, int):
