@@ -657,20 +657,21 @@ int hh_act_tiles_launch(int fmt, const uint8_t* x, const int8_t* xq, const float
 // int8, 10.4 straight from the blocks, the form chosen here.  Of the products from K =
 // 1024 int8 keeps one corner, PTQ1_0 12288 x 1024 at 96 and 128 tokens: 14.3, here 15.6.)
 enum : int { F4_TILE, F4_ROWS, X_128x64_8, X_128x64_4, X_128x128, X_256x128, N_FORMS };
-constexpr int FORM_ROWS[N_FORMS] = {32, 128, 128, 128, 128, 256};
-constexpr int FORM_GROUPS[N_FORMS] = {1, 1, 2, 2, 4, 4};   // 32-token groups
+constexpr int FORM_ROWS[N_FORMS] = {5, 7, 7, 7, 7, 8};     // log2 rows and
+constexpr int FORM_GROUPS[N_FORMS] = {0, 0, 1, 1, 2, 2};   // 32-token groups per workgroup
 
 // us of one pass over n rows in a form (the expanded ones without their expansion).
 static double form_us(int form, int fmt, int n, int K, int ng) {
-  const long g = (long)((n + FORM_ROWS[form] - 1) / FORM_ROWS[form]) * ((ng + FORM_GROUPS[form] - 1) / FORM_GROUPS[form]);
-  const double u = K / 128;
-  const double waves = (double)((g + 255) / 256);               // rounds at one workgroup per CU
-  const double pairs = (double)(g / 512 + (g % 512 > 256));     // at two, but for
-  const double tail = g % 512 != 0 && g % 512 <= 256;           // a last one of one per CU
+  const int rl = FORM_ROWS[form], gl = FORM_GROUPS[form];
+  const long g = (long)((n + (1 << rl) - 1) >> rl) * ((ng + (1 << gl) - 1) >> gl);
+  const double u = K >> 7;
+  const double waves = (double)((g + 255) >> 8);                // rounds at one workgroup per CU
+  const double pairs = (double)((g >> 9) + ((g & 511) > 256));  // at two, but for
+  const double tail = (g & 511) != 0 && (g & 511) <= 256;       // a last one of one per CU
   switch (form) {
     case F4_TILE: {   // 16 column blocks are one memory round trip
       const double trip = fmt == FMT_Q1 ? 3.6 : fmt == FMT_Q2 ? 4.0 : 4.7;
-      return 1.1 + waves * trip * ((K + 2047) / 2048);
+      return 1.1 + waves * trip * ((K + 2047l) >> 11);
     }
     case F4_ROWS:   // unpacks its weights in every workgroup: by format
       if (fmt == FMT_Q1) return 2.8 + (g <= 256 ? 0.64 * u : pairs * (0.18 + 0.77 * u) + tail * 0.435 * u);
@@ -691,52 +692,57 @@ static int slab_rows(int n, int K) {   // rows per expansion: whole 256-row tile
   return (int)std::min<size_t>((n + 255) / 256, std::max<size_t>(1, F4X_SLAB / per)) * 256;
 }
 static double expand_us(int n, int K) { return 2.0 + 0.16e-6 * n * K; }
-static int best_expanded(int fmt, int n, int K, int ng) {
+static int best_expanded(int fmt, int n, int K, int ng, double* us) {
   int best = X_128x64_8;
-  for (int f = best + 1; f < N_FORMS; ++f)
-    if (form_us(f, fmt, n, K, ng) < form_us(best, fmt, n, K, ng)) best = f;
+  *us = form_us(best, fmt, n, K, ng);
+  for (int f = best + 1; f < N_FORMS; ++f) {
+    const double t = form_us(f, fmt, n, K, ng);
+    if (t < *us) { *us = t; best = f; }
+  }
   return best;
 }
 
 // The form without expanded weights, and the one that is chosen (for the first slab).
-static int direct_form(int fmt, int n, int K, int ng) {
+static int direct_form(int fmt, int n, int K, int ng, double* us) {
+  *us = form_us(F4_ROWS, fmt, n, K, ng);
   // past 16 rounds the row form always wins
   if ((long)((n + 31) / 32) * ng > 4096) return F4_ROWS;
-  return form_us(F4_TILE, fmt, n, K, ng) < form_us(F4_ROWS, fmt, n, K, ng) ? F4_TILE : F4_ROWS;
+  const double tile = form_us(F4_TILE, fmt, n, K, ng);
+  if (!(tile < *us)) return F4_ROWS;
+  *us = tile;
+  return F4_TILE;
 }
-static int choose_form(int fmt, int n, int K, int seq) {
-  const int ng = (seq + 31) / 32, direct = direct_form(fmt, n, K, ng);
+
+int hh_gemm_f4_form(int fmt, int n, int K, int seq) {
+  const int ng = (seq + 31) / 32;
+  double limit, us = 0.0, t;
+  const int direct = direct_form(fmt, n, K, ng, &limit);
   if (ng < 2) return direct;   // one group leaves half of every expanded tile empty
   // (a grid dimension holds 2^32 lanes: the row form's tiles may be more)
-  const bool fits = (long)((n + 127) / 128) * ng < (1l << 24);
-  const double limit = fits ? form_us(direct, fmt, n, K, ng) : 1e30;
+  if ((long)((n + 127) / 128) * ng >= (1l << 24)) limit = 1e30;
   const int slab = slab_rows(n, K);
-  double us = 0.0;
+  int first = -1;
   for (int r0 = 0; r0 < n && us < limit; r0 += slab) {
-    const int nr = std::min(slab, n - r0);
-    us += expand_us(nr, K) + form_us(best_expanded(fmt, nr, K, ng), fmt, nr, K, ng);
+    const int nr = std::min(slab, n - r0), f = best_expanded(fmt, nr, K, ng, &t);
+    if (first < 0) first = f;
+    us += expand_us(nr, K) + t;
   }
-  return us < limit ? best_expanded(fmt, std::min(slab, n), K, ng) : direct;
+  return us < limit ? first : direct;
 }
 
-// The chosen form and its rows per pass (fewer than n: expanded in slabs).
-int hh_gemm_f4_plan(int fmt, int n, int K, int seq, int* rows) {
-  const int form = choose_form(fmt, n, K, seq);
-  *rows = form >= X_128x64_8 ? std::min(slab_rows(n, K), n) : n;
-  return form;
+int hh_gemm_f4_pass_rows(int form, int n, int K) { return form >= X_128x64_8 ? std::min(slab_rows(n, K), n) : n; }
+
+size_t hh_gemm_f4_wbytes(int form, int n, int K) {
+  return form >= X_128x64_8 ? (size_t)(slab_rows(n, K) / 32) * (K / 128) * WT_BYTES : 0;
 }
 
-size_t hh_gemm_f4_wbytes(int fmt, int n, int K, int seq) {
-  return choose_form(fmt, n, K, seq) >= X_128x64_8 ? (size_t)(slab_rows(n, K) / 32) * (K / 128) * WT_BYTES : 0;
-}
-
-int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* tiles, int seq, uint8_t* wtiles,
-                      float* out, hipStream_t s) {
+int hh_gemm_f4_launch(int fmt, int form, const uint8_t* w, int n, int K, const uint8_t* tiles, int seq,
+                      uint8_t* wtiles, float* out, hipStream_t s) {
   if (K <= 0 || K % 128 != 0 || n <= 0 || seq <= 0 || (fmt != FMT_Q2 && fmt != FMT_Q1 && fmt != FMT_PT)) return 1;
   const int ng = (seq + 31) / 32, ngp = act_groups(seq);
   const int vec = n % 4 == 0 && ((uintptr_t)out & 15) == 0;
-  int form = choose_form(fmt, n, K, seq);
-  if (form >= X_128x64_8 && !wtiles) form = direct_form(fmt, n, K, ng);
+  double us;
+  if (form >= X_128x64_8 && !wtiles) form = direct_form(fmt, n, K, ng, &us);
   if (form < X_128x64_8) {
     const bool small = form == F4_TILE;
     const dim3 grid(small ? (unsigned)((n + 31) / 32) * ng : (unsigned)((n + 127) / 128) * ng);
@@ -765,7 +771,7 @@ int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* ti
   hipLaunchKernelGGL((k_gemm_f4x<RT, TT, WR, WT, NS>),                                                           \
                      dim3((nr + 32 * RT * WR - 1) / (32 * RT * WR), (ng + TT * WT - 1) / (TT * WT)),             \
                      dim3(64 * WR * WT), 0, s, wtiles, tiles, out, r0, n, K, seq, rg, ngp, vec)
-    switch (best_expanded(fmt, nr, K, ng)) {
+    switch (best_expanded(fmt, nr, K, ng, &us)) {
       case X_128x64_8: HH_F4X(1, 1, 4, 2, 4); break;
       case X_128x64_4: HH_F4X(2, 1, 2, 2, 3); break;
       case X_128x128: HH_F4X(2, 2, 2, 2, 2); break;

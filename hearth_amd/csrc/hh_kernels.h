@@ -150,13 +150,13 @@ constexpr int HH_ACT_TILE_BYTES = 6656;
 size_t hh_act_tiles_bytes(int K, int seq);
 int hh_act_tiles_launch(int fmt, const uint8_t* x, const int8_t* xq, const float* xd, int K, int seq, uint8_t* tiles,
                         hipStream_t s);
-// wtiles: hh_gemm_f4_wbytes(fmt, n, K, seq) bytes of scratch for expanded weights (null:
-// not used, slower where that is not 0); hh_gemm_f4_plan: the form of the product (0 32 x
-// 32 tiles, 1 128 x 32, 2 .. 5 expanded: 128 x 64 by 8 and 4 waves, 128 x 128, 256 x 128)
-// and its rows per pass
-int hh_gemm_f4_plan(int fmt, int n, int K, int seq, int* rows);
-size_t hh_gemm_f4_wbytes(int fmt, int n, int K, int seq);
-int hh_gemm_f4_launch(int fmt, const uint8_t* w, int n, int K, const uint8_t* tiles, int seq, uint8_t* wtiles,
+// form: hh_gemm_f4_form's (0 32 x 32 tiles, 1 128 x 32, 2 .. 5 expanded: 128 x 64 by 8 and 4
+// waves, 128 x 128, 256 x 128); wtiles: hh_gemm_f4_wbytes(form, n, K) bytes of scratch for
+// expanded weights (null: not used, slower where that is not 0)
+int hh_gemm_f4_form(int fmt, int n, int K, int seq);
+int hh_gemm_f4_pass_rows(int form, int n, int K);   // rows expanded at a time
+size_t hh_gemm_f4_wbytes(int form, int n, int K);
+int hh_gemm_f4_launch(int fmt, int form, const uint8_t* w, int n, int K, const uint8_t* tiles, int seq, uint8_t* wtiles,
                       float* out, hipStream_t s);
 
 int hh_quantize_launch(const float* x, int64_t n, uint8_t* out, hipStream_t s);

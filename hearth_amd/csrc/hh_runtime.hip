@@ -599,7 +599,7 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
   for (const Layer& L : m->layers) n_in_max = std::max(n_in_max, L.n_in);
   const int kmax = std::max(std::max(d, F), std::max(nq, vdim));
   size_t wt_max = 0;   // expanded weights of the largest projection that wants them
-  auto with = [&](int n, int K) { wt_max = std::max(wt_max, hh_gemm_f4_wbytes(m->wfmt, n, K, S)); };
+  auto with = [&](int n, int K) { wt_max = std::max(wt_max, hh_gemm_f4_wbytes(hh_gemm_f4_form(m->wfmt, n, K, S), n, K)); };
   for (const Layer& L : m->layers) {
     with(L.n_in, d);
     with(d, L.gdn ? vdim : nq);
@@ -656,7 +656,8 @@ int prefill_batched(hh_model* m, const uint32_t* toks, int S, int pos0) {
       const float* xd = Xd + (size_t)t0 * (K / 32);
       if (const int rc = hh_act_tiles_launch(m->wfmt, nullptr, xq, xd, K, nt, Act, s)) return rc;
       uint8_t* wt = expand && wt_max ? Act + act : nullptr;
-      if (const int rc = hh_gemm_f4_launch(m->wfmt, w, n, K, Act, nt, wt, out + (size_t)t0 * n, s)) return rc;
+      const int form = hh_gemm_f4_form(m->wfmt, n, K, nt);
+      if (const int rc = hh_gemm_f4_launch(m->wfmt, form, w, n, K, Act, nt, wt, out + (size_t)t0 * n, s)) return rc;
     }
     return 0;
   };
@@ -914,11 +915,11 @@ static int gemm_args(int type, int64_t n_rows, int64_t n_cols, int64_t seq_len, 
 
 int hh_gemm_q8_plan(int type, int64_t n_rows, int64_t n_cols, int64_t seq_len, int* form, int64_t* rows_per_pass) {
   if (!form || !rows_per_pass) return fail(HH_ERR_INVALID, "null argument");
-  int fmt, rows = (int)n_rows;
+  int fmt;
   const int rc = gemm_args(type, n_rows, n_cols, seq_len, &fmt);
   if (rc != HH_OK) return rc;
-  *form = fmt == FMT_Q8 ? 6 : hh_gemm_f4_plan(fmt, (int)n_rows, (int)n_cols, (int)seq_len, &rows);
-  *rows_per_pass = rows;
+  *form = fmt == FMT_Q8 ? 6 : hh_gemm_f4_form(fmt, (int)n_rows, (int)n_cols, (int)seq_len);
+  *rows_per_pass = fmt == FMT_Q8 ? n_rows : hh_gemm_f4_pass_rows(*form, (int)n_rows, (int)n_cols);
   return HH_OK;
 }
 
@@ -942,7 +943,8 @@ int hh_gemm_q8(hh_ctx* c, int type, const void* w, int64_t n_rows, int64_t n_col
     KTRY(hh_gemm_launch((const uint8_t*)w, n, K, xq, xd, S, out, c->stream));
     return HH_OK;
   }
-  const size_t wt = hh_gemm_f4_wbytes(fmt, n, K, S);
+  const int form = hh_gemm_f4_form(fmt, n, K, S);
+  const size_t wt = hh_gemm_f4_wbytes(form, n, K);
   int ST = S;   // tokens per pass
   bool expand = true;
   size_t act = 0;
@@ -957,8 +959,8 @@ int hh_gemm_q8(hh_ctx* c, int type, const void* w, int64_t n_rows, int64_t n_col
   for (int t0 = 0; t0 < S; t0 += ST) {
     const int nt = std::min(ST, S - t0);
     KTRY(hh_act_tiles_launch(fmt, xq8 + (size_t)t0 * (K / 32) * 34, nullptr, nullptr, K, nt, buf, c->stream));
-    KTRY(hh_gemm_f4_launch(fmt, (const uint8_t*)w, n, K, buf, nt, expand && wt ? buf + act : nullptr,
-                           out + (size_t)t0 * n, c->stream));
+    KTRY(hh_gemm_f4_launch(fmt, nt == S ? form : hh_gemm_f4_form(fmt, n, K, nt), (const uint8_t*)w, n, K, buf, nt,
+                           expand && wt ? buf + act : nullptr, out + (size_t)t0 * n, c->stream));
   }
   return HH_OK;
 }
