@@ -647,15 +647,18 @@ int hh_act_tiles_launch(int fmt, const uint8_t* x, const int8_t* xq, const float
 }
 
 // The forms of a product and the time each takes, from which the launcher chooses.
-// A form costs a start, and for each of its rounds (the workgroups that fit the 256
-// CUs at once) a fixed part and a part per 128 columns.  The figures are fits to 2829
-// measured products (K 128 .. 17408, 1024 .. 34816 rows, 2 .. 2048 tokens, the three
-// formats, weights cold), where the choice by them takes 0.1% longer than the fastest
-// form on average and, from K = 1024, 10% at most.  (Thresholds on the tokens and the
-// grid alone, set at K = 4096, took up to 57% longer, and at K = 1024 longer than an int8
+// A form costs a start, its workgroups' loads and stores against each other, and for
+// each of its rounds (the workgroups that fit the 256 CUs at once) a fixed part and a
+// part per 128 columns.  The figures are fits to 6153 measured products (K 128 ..
+// 17408, 1024 .. 34816 rows, 2 .. 2048 tokens, the three formats, weights cold); the
+// choice by them takes 0.1% longer than the fastest form on average, and 17% at most
+// from K = 1024 (more than 5% in 25 of 5082).  (Thresholds on the tokens and the grid
+// alone, set at K = 4096, took up to 57% longer, and at K = 1024 longer than an int8
 // MFMA kernel: Q2_0, 6144 x 1024, 224 tokens 13.2 us expanded in 128 x 64 tiles, 12.3
-// int8, 10.4 straight from the blocks, the form chosen here.  Of the products from K =
-// 1024 int8 keeps one corner, PTQ1_0 12288 x 1024 at 96 and 128 tokens: 14.3, here 15.6.)
+// int8, 10.4 straight from the blocks, the form chosen here.  int8 keeps one corner,
+// PTQ1_0 of some 8192 .. 16384 rows at 65 .. 256 tokens with K 1024 .. 1536, where no
+// form here reaches it, by 2 to 9%: 16384 x 1024, 128 tokens 14.8, here 15.5; and with
+// 16384 rows and K = 17408, past one slab, 187, here 207.)
 enum : int { F4_TILE, F4_ROWS, X_128x64_8, X_128x64_4, X_128x128, X_256x128, N_FORMS };
 constexpr int FORM_ROWS[N_FORMS] = {5, 7, 7, 7, 7, 8};     // log2 rows and
 constexpr int FORM_GROUPS[N_FORMS] = {0, 0, 1, 1, 2, 2};   // 32-token groups per workgroup
@@ -664,23 +667,25 @@ constexpr int FORM_GROUPS[N_FORMS] = {0, 0, 1, 1, 2, 2};   // 32-token groups pe
 static double form_us(int form, int fmt, int n, int K, int ng) {
   const int rl = FORM_ROWS[form], gl = FORM_GROUPS[form];
   const long g = (long)((n + (1 << rl) - 1) >> rl) * ((ng + (1 << gl) - 1) >> gl);
-  const double u = K >> 7;
+  const double u = K >> 7, r = g * (1.0 / 512);
   const double waves = (double)((g + 255) >> 8);                // rounds at one workgroup per CU
   const double pairs = (double)((g >> 9) + ((g & 511) > 256));  // at two, but for
   const double tail = (g & 511) != 0 && (g & 511) <= 256;       // a last one of one per CU
   switch (form) {
     case F4_TILE: {   // 16 column blocks are one memory round trip
-      const double trip = fmt == FMT_Q1 ? 3.6 : fmt == FMT_Q2 ? 4.0 : 4.7;
-      return 1.1 + waves * trip * ((K + 2047l) >> 11);
+      const double trip = fmt == FMT_Q1 ? 3.65 : fmt == FMT_Q2 ? 3.99 : 4.39;
+      return 1.2 + waves * trip * ((K + 2047l) >> 11);
     }
     case F4_ROWS:   // unpacks its weights in every workgroup: by format
-      if (fmt == FMT_Q1) return 2.8 + (g <= 256 ? 0.64 * u : pairs * (0.18 + 0.77 * u) + tail * 0.435 * u);
-      if (fmt == FMT_Q2) return 2.5 + (g <= 256 ? 0.74 * u : pairs * (0.2 + 0.925 * u) + tail * 0.52 * u);
-      return 2.0 + (g <= 256 ? 1.24 * u : 0.26 * u + pairs * (0.4 + 1.33 * u) + tail * 0.5 * u);
-    case X_128x64_8: return 0.9 + waves * (4.3 + 0.54 * u);
-    case X_128x64_4: return 3.7 + tail * (1.4 + 0.63 * u) + pairs * (5.6 + 0.946 * u);
-    case X_128x128: return 3.7 + tail * (1.4 + 1.11 * u) + pairs * (5.6 + 1.777 * u);
-    default: return waves * (11.3 + 1.68 * u);
+      if (fmt == FMT_Q1)
+        return 2.118 + 0.89 * r + (g <= 256 ? 0.7 * u : 0.116 * u + pairs * 0.707 * u + tail * 0.393 * u);
+      if (fmt == FMT_Q2)
+        return 2.2 + 1.1 * r + (g <= 256 ? 0.745 * u : 0.084 * u + pairs * 0.828 * u + tail * 0.432 * u);
+      return 1.251 + 1.474 * r + (g <= 256 ? 1.301 * u : 0.443 * u + pairs * 1.09 * u + tail * 0.519 * u);
+    case X_128x64_8: return 3.277 + 6.4 * r + waves * (0.721 + 0.535 * u);
+    case X_128x64_4: return 4.234 + 4.454 * r + tail * 0.612 * u + pairs * (1.2 + 0.963 * u);
+    case X_128x128: return 4.053 + 6.65 * r + tail * 1.123 * u + pairs * 1.774 * u;
+    default: return 5.922 + 18.534 * r + waves * (3.41 + 1.673 * u);
   }
 }
 
@@ -691,7 +696,7 @@ static int slab_rows(int n, int K) {   // rows per expansion: whole 256-row tile
   const size_t per = (size_t)(K / 128) * 8 * WT_BYTES;
   return (int)std::min<size_t>((n + 255) / 256, std::max<size_t>(1, F4X_SLAB / per)) * 256;
 }
-static double expand_us(int n, int K) { return 2.0 + 0.16e-6 * n * K; }
+static double expand_us(int n, int K) { return 2.223 + 0.161e-6 * n * K; }
 static int best_expanded(int fmt, int n, int K, int ng, double* us) {
   int best = X_128x64_8;
   *us = form_us(best, fmt, n, K, ng);

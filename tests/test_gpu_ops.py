@@ -359,19 +359,19 @@ FORMS = [
     (0, 42, 1023, 2176, 33, None), (0, 41, 257, 4224, 65, None), (0, 143, 127, 6016, 31, None),
     # 128 x 32 straight from the blocks, 8 and 7 steps through its two buffers
     (1, 41, 12289, 1024, 33, None), (1, 42, 12289, 1024, 33, None), (1, 143, 12289, 896, 33, None),
-    # expanded, 128 x 64 by 8 waves (ring of 4): 18 .. 20 and 23 steps
-    (2, 143, 4097, 2304, 33, None), (2, 143, 4097, 2432, 33, None), (2, 143, 4097, 2560, 33, None),
-    (2, 41, 2049, 2944, 511, None), (2, 42, 2049, 2176, 511, None),
-    # 128 x 64 by 4 waves (ring of 3): 5 .. 7 and 15 steps
-    (3, 143, 12289, 640, 257, None), (3, 143, 16385, 768, 161, None), (3, 143, 16385, 896, 161, None),
-    (3, 42, 16385, 1920, 161, None),
-    # 128 x 128 (ring of 2): 6, 7, 8 and 11 steps
-    (4, 143, 6145, 768, 333, None), (4, 143, 12289, 896, 161, None), (4, 42, 2049, 1024, 1500, None),
-    (4, 41, 2049, 1408, 1500, None),
-    # 256 x 128 (ring of 3): 21 .. 23 steps
-    (5, 42, 24577, 2688, 200, None), (5, 143, 24577, 2816, 200, None), (5, 42, 24577, 2944, 200, None),
+    # expanded, 128 x 64 by 8 waves (ring of 4): 8, 17 .. 19, 23 and 30 steps
+    (2, 143, 2049, 1024, 257, None), (2, 143, 4097, 2176, 33, None), (2, 143, 4097, 2304, 33, None),
+    (2, 143, 4097, 2432, 33, None), (2, 41, 2049, 2944, 511, None), (2, 42, 2049, 3840, 257, None),
+    # 128 x 64 by 4 waves (ring of 3): 7 .. 9 and 13 steps
+    (3, 143, 16385, 896, 161, None), (3, 143, 6145, 1024, 257, None), (3, 143, 6145, 1152, 257, None),
+    (3, 42, 8193, 1664, 400, None),
+    # 128 x 128 (ring of 2): 4, 7, 9 and 10 steps
+    (4, 143, 2049, 512, 1500, None), (4, 143, 6145, 896, 333, None), (4, 41, 6145, 1152, 1000, None),
+    (4, 42, 2049, 1280, 1500, None),
+    # 256 x 128 (ring of 3): 96 .. 98 steps
+    (5, 42, 14840, 12288, 400, None), (5, 143, 14839, 12416, 400, None), (5, 42, 14593, 12544, 385, None),
     # the weights expanded in slabs, the last of 153, 257 and (a third) 257 rows
-    (2, 143, 15001, 17408, 96, 14848), (5, 42, 15105, 17408, 400, 14848), (3, 143, 29953, 17408, 129, 14848)]
+    (2, 143, 15001, 17408, 96, 14848), (5, 42, 15105, 17408, 400, 14848), (3, 143, 29953, 17408, 161, 14848)]
 
 
 @pytest.mark.parametrize("form,t,n,k,seq,slab", FORMS)
